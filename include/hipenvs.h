@@ -389,6 +389,16 @@ int hipenvs_div_recip(const float* a, const float* d, float* q, uint8_t* marked,
 int hipenvs_sqrt_recip_check(uint64_t first, uint64_t count, unsigned long long* counts,
                              hipenvs_stream_t stream);
 
+/* For every float32 bit pattern first .. first + count - 1 (within 0 .. 2^32 - 1), the
+ * kernels' shortened arithmetic: adds to counts[0] the inputs whose tanh differs from the
+ * same polynomial with every product rounded and IEEE division, to counts[1] those (|x| <=
+ * 256) whose sin/cos argument reduction differs from the unfused one, to counts[2] the
+ * positive normals whose Cholesky pivot root differs from IEEE sqrtf, and to counts[3] those
+ * (below 2^126) whose float64 pivot or divisor reciprocal is off by more than 2^-51. counts:
+ * four values of device memory the caller zeroes. */
+int hipenvs_arith_check(uint64_t first, uint64_t count, unsigned long long* counts,
+                        hipenvs_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -53,6 +53,63 @@ __global__ __launch_bounds__(kBlock) void sqrt_recip_check_kernel(uint64_t first
   if (!r_ok) atomicAdd(&counts[1], 1ull);
 }
 
+// The plain forms of det_tanh and of the float32 reduction: every product rounded on its own,
+// IEEE division.
+__device__ __forceinline__ float tanh_plain(float x) {
+  float a = fabsf(x);
+  a = (a > dm::TANH_CLAMP) ? dm::TANH_CLAMP : a;
+  const float y = a + a;
+  const float k = rintf(y * dm::LOG2E);
+  const float r = (y - k * dm::LN2_HI) - k * dm::LN2_LO;
+  float p = dm::E7 + r * dm::E8;
+  p = dm::E6 + r * p;
+  p = dm::E5 + r * p;
+  p = dm::E4 + r * p;
+  p = dm::E3 + r * p;
+  p = dm::E2 + r * p;
+  p = r + (r * r) * p;
+  const int ki = (k >= 0.0f && k <= 64.0f) ? (int)k : 0;
+  const float two_k = __int_as_float((ki + 127) << 23);
+  const float e = two_k * p + (two_k - 1.0f);
+  const float t = e / (e + 2.0f);
+  return copysignf(t, x);
+}
+
+__device__ __forceinline__ float reduce_plain(float x, int* q) {
+  const float k = rintf(x * dm::TWO_OVER_PI);
+  *q = (int)k;
+  return (((x - k * dm::PIO2_1) - k * dm::PIO2_2) - k * dm::PIO2_3) - k * dm::PIO2_4;
+}
+
+__device__ __forceinline__ bool same_bits(float a, float b) {
+  return __float_as_uint(a) == __float_as_uint(b) || (a != a && b != b);
+}
+
+// Every float32 bit pattern first + i, i < count: counts[0] det_tanh against its plain form,
+// counts[1] the float32 argument reduction against its plain form (|x| <= 256), counts[2]
+// sqrt_pivot's root against IEEE sqrtf (positive normals), counts[3] its reciprocal and
+// recip_normal's against 1 / x in float64, beyond 2^-51 relative (positive normals below 2^126).
+__global__ __launch_bounds__(kBlock) void arith_check_kernel(uint64_t first, uint64_t count,
+                                                             unsigned long long* __restrict__ counts) {
+  const uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= count) return;
+  const float x = __uint_as_float((uint32_t)(first + i));
+  if (!same_bits(det_tanh(x), tanh_plain(x))) atomicAdd(&counts[0], 1ull);
+  if (fabsf(x) <= dm::SMALL_ARG) {
+    int qa, qb;
+    const float ra = reduce_small(x, &qa), rb = reduce_plain(x, &qb);
+    if (!same_bits(ra, rb) || qa != qb) atomicAdd(&counts[1], 1ull);
+  }
+  if (x >= 0x1p-126f && x < 0x1p+126f) {
+    double r;
+    const float y = sqrt_pivot(x, &r);
+    if (!same_bits(y, sqrtf(x))) atomicAdd(&counts[2], 1ull);
+    const double e_root = fabs(__builtin_fma(-(double)y, r, 1.0));
+    const double e_recip = fabs(__builtin_fma(-(double)x, recip_normal(x), 1.0));
+    if (!(e_root <= 0x1p-51) || !(e_recip <= 0x1p-51)) atomicAdd(&counts[3], 1ull);
+  }
+}
+
 }  // namespace diag
 }  // namespace hipenvs
 
@@ -81,6 +138,15 @@ extern "C" int hipenvs_sqrt_recip_check(uint64_t first, uint64_t count, unsigned
   if (!counts || first > 0xFFFFFFFFull || count > (1ull << 32) - first) return HIPENVS_E_ARG;
   if (count == 0) return HIPENVS_OK;
   hipLaunchKernelGGL(diag::sqrt_recip_check_kernel, dim3((unsigned)((count + kBlock - 1) / kBlock)), dim3(kBlock), 0,
+                     as_stream(stream), first, count, counts);
+  return launch_status();
+}
+
+extern "C" int hipenvs_arith_check(uint64_t first, uint64_t count, unsigned long long* counts,
+                                   hipenvs_stream_t stream) {
+  if (!counts || first > 0xFFFFFFFFull || count > (1ull << 32) - first) return HIPENVS_E_ARG;
+  if (count == 0) return HIPENVS_OK;
+  hipLaunchKernelGGL(diag::arith_check_kernel, dim3((unsigned)((count + kBlock - 1) / kBlock)), dim3(kBlock), 0,
                      as_stream(stream), first, count, counts);
   return launch_status();
 }

@@ -94,14 +94,33 @@ __device__ __forceinline__ void sincos_poly(float r, float* sin_out, float* cos_
   *cos_out = 1.0f + z * cp;
 }
 
+// The float32 reduction of |x| <= 256 to r in [-pi/4, pi/4] and the quadrant in q's low two
+// bits. k * PIO2_1..3 are exact (a 12-bit piece, |k| <= 163), so each fused multiply-add
+// rounds x - k * piece once, as the separate multiply and subtract do: the same bits in three
+// fewer instructions. The last piece's product is inexact and stays separate.
+__device__ __forceinline__ float reduce_small(float x, int* q) {
+  const float k = rintf(x * dm::TWO_OVER_PI);
+  *q = (int)k;
+  const float r = __builtin_fmaf(-k, dm::PIO2_3, __builtin_fmaf(-k, dm::PIO2_2, __builtin_fmaf(-k, dm::PIO2_1, x)));
+  return r - k * dm::PIO2_4;
+}
+
+// sin and cos from the reduced argument: the polynomials, then the quadrant's swap and signs.
+__device__ __forceinline__ void sincos_quadrant(float r, int q, float* sin_out, float* cos_out) {
+  float s, c;
+  sincos_poly(r, &s, &c);
+  const float a = (q & 1) ? c : s;
+  const float b = (q & 1) ? s : c;
+  *sin_out = (q & 2) ? -a : a;
+  *cos_out = ((q + 1) & 2) ? -b : b;
+}
+
 __device__ __forceinline__ void det_sincos(float x, float* sin_out, float* cos_out) {
   // float32 reduction, computed for every lane on an argument clamped into its range (so
   // no branch precedes it and independent work can overlap the loads that feed x) ...
   const bool small = fabsf(x) <= dm::SMALL_ARG;
-  const float xs = small ? x : 0.0f;
-  const float k = rintf(xs * dm::TWO_OVER_PI);
-  float r = (((xs - k * dm::PIO2_1) - k * dm::PIO2_2) - k * dm::PIO2_3) - k * dm::PIO2_4;
-  int q = (int)k & 3;
+  int q;
+  float r = reduce_small(small ? x : 0.0f, &q);
   if (!small) {  // ... and the float64 reduction for |x| > 256, inf and NaN
     const double xd = (double)x;
     const double kd = rint(xd * dm::TWO_OVER_PI_D);
@@ -109,12 +128,28 @@ __device__ __forceinline__ void det_sincos(float x, float* sin_out, float* cos_o
     const double qd = kd - 4.0 * floor(kd * 0.25);
     q = (qd >= 0.0 && qd < 4.0) ? ((int)qd & 3) : 0;  // inf/NaN: quadrant 0, result NaN
   }
-  float s, c;
-  sincos_poly(r, &s, &c);
-  const float a = (q & 1) ? c : s;
-  const float b = (q & 1) ? s : c;
-  *sin_out = (q & 2) ? -a : a;
-  *cos_out = ((q + 1) & 2) ? -b : b;
+  sincos_quadrant(r, q, sin_out, cos_out);
+}
+
+// det_sincos of K arguments under one wave vote: when every active lane has all K of them
+// within 256 (always, for wrapped angles) the float32 reductions alone, with no branch
+// between them, so the K streams interleave; det_sincos of each otherwise.
+template <int K>
+__device__ __forceinline__ void det_sincos_small(const float (&x)[K], float (&sin_out)[K], float (&cos_out)[K]) {
+  bool ok = true;
+#pragma unroll
+  for (int i = 0; i < K; ++i) ok &= fabsf(x[i]) <= dm::SMALL_ARG;
+  if (__all(ok)) {
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      int q;
+      const float r = reduce_small(x[i], &q);
+      sincos_quadrant(r, q, &sin_out[i], &cos_out[i]);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < K; ++i) det_sincos(x[i], &sin_out[i], &cos_out[i]);
+  }
 }
 
 // Deterministic float64 sin/cos, for the reference-precision legged step (the reference's
@@ -242,12 +277,24 @@ __device__ __forceinline__ float det_cos(float x) {
   return c;
 }
 
+// det_tanh in the fewest instructions that give its bits (33 where the plain form takes about
+// 48; one of the 64 units of a policy layer each step, so it bounds the CartPole and Acrobot
+// rollouts):
+// - rint(y log2 e) by adding and subtracting 1.5 * 2^23, which rounds the product to an integer
+//   the same way and leaves it in the sum's low bits, whence 2^k by one shift-add (a NaN's
+//   garbage power meets a NaN polynomial);
+// - k * LN2_HI (16-bit head, k <= 29) and 2^k * p are exact, so the fused forms round once as
+//   the separate ones do;
+// - e / (e + 2) from the reciprocal estimate and one residual correction, equal to the IEEE
+//   quotient for each of the 2^32 inputs (hipenvs_arith_check, run by the GPU tests).
 __device__ __forceinline__ float det_tanh(float x) {
+  constexpr float kRound = 0x1.8p+23f;
   float a = fabsf(x);
   a = (a > dm::TANH_CLAMP) ? dm::TANH_CLAMP : a;  // NaN compares false and stays NaN
   const float y = a + a;
-  const float k = rintf(y * dm::LOG2E);
-  const float r = (y - k * dm::LN2_HI) - k * dm::LN2_LO;
+  const float t = y * dm::LOG2E + kRound;
+  const float k = t - kRound;
+  const float r = __builtin_fmaf(-k, dm::LN2_HI, y) - k * dm::LN2_LO;
   float p = dm::E7 + r * dm::E8;
   p = dm::E6 + r * p;
   p = dm::E5 + r * p;
@@ -255,11 +302,12 @@ __device__ __forceinline__ float det_tanh(float x) {
   p = dm::E3 + r * p;
   p = dm::E2 + r * p;
   p = r + (r * r) * p;
-  const int ki = (k >= 0.0f && k <= 64.0f) ? (int)k : 0;
-  const float two_k = __int_as_float((ki + 127) << 23);
-  const float e = two_k * p + (two_k - 1.0f);
-  const float t = e / (e + 2.0f);
-  return copysignf(t, x);
+  const float two_k = __uint_as_float((__float_as_uint(t) << 23) + 0x3F800000u);
+  const float e = __builtin_fmaf(two_k, p, two_k - 1.0f);
+  const float d = e + 2.0f;
+  const float rd = __builtin_amdgcn_rcpf(d);
+  const float q = e * rd;
+  return copysignf(__builtin_fmaf(__builtin_fmaf(-q, d, e), rd, q), x);
 }
 
 // x / c for a float32 constant c, as one float64 product with inv_c = 1 / (double)c
@@ -310,6 +358,37 @@ __device__ __forceinline__ float sqrt_rn(float x) {
   const double e = __builtin_fma(-g, g, d);
   const float y = (float)__builtin_fma(0.5 * r, e, g);
   return __builtin_amdgcn_classf(x, 0x260) ? x : y;  // class bits 5, 6, 9: -0, +0, +inf
+}
+
+// Float64 reciprocal of a float32 d that is normal and finite (or NaN, which stays NaN) for
+// DivRecip: the hardware estimate r0 and one third-order step,
+// r0 + r0 (e + e^2) with e = 1 - d r0 (|e| < 2^-20, so the truncation is below 2^-60 and the
+// result is within an ulp of 1 / d). Five instructions where recip() takes nine: a quotient
+// needs the reciprocal only to well within 2^-50 (see above), not correctly rounded, and these
+// divisors are never 0 or infinite.
+__device__ __forceinline__ double recip_normal(float d) {
+  const double x = (double)d;
+  const double r0 = __builtin_amdgcn_rcp(x);
+  const double e = __builtin_fma(-x, r0, 1.0);
+  return __builtin_fma(r0, __builtin_fma(e, e, e), r0);
+}
+
+// The square root y = sqrtf(s) of a Cholesky pivot and the float64 reciprocal of y, for s
+// normal, finite and positive (or NaN). The mass matrices here depend on the angles alone
+// through their sines and cosines and are positive definite over that compact set, the smallest
+// pivot 0.0625 (legged) and 0.5 (pendulum), so s is never 0 or infinite. y is sqrt_rn without its
+// special cases; its reciprocal starts from the same estimate r of 1 / sqrt(s) (y differs
+// from sqrt(s) by half an ulp, so 1 - y r is below 2^-20) and takes one third-order step. Eleven
+// instructions and one transcendental where sqrt_rn and recip take eighteen and two.
+__device__ __forceinline__ float sqrt_pivot(float s, double* recip_out) {
+  const double d = (double)s;
+  const double r = __builtin_amdgcn_rsq(d);
+  const double g = d * r;
+  const double e = __builtin_fma(-g, g, d);
+  const float y = (float)__builtin_fma(0.5 * r, e, g);
+  const double f = __builtin_fma(-(double)y, r, 1.0);
+  *recip_out = __builtin_fma(r, __builtin_fma(f, f, f), r);
+  return y;
 }
 
 struct DivRecip {

@@ -94,7 +94,7 @@ __device__ __forceinline__ void accelerations_with(const float* th, const float*
       uu[i] = (i == 0 ? torque : 0.0f) - P0;
       if (i == 0) break;
       const float D = A0;
-      const double rD = recip(D);
+      const double rD = recip_normal(D);  // D >= 1: a link's own inertia plus what it carries
       const float I0 = A0 - div(A0 * A0, D, rD), I1 = A1 - div(A0 * A1, D, rD), I2 = A2 - div(A0 * A2, D, rD);
       const float I3 = A3 - div(A1 * A1, D, rD), I4 = A4 - div(A1 * A2, D, rD), I5 = A5 - div(A2 * A2, D, rD);
       const float qd = om[i] - om[i - 1];
@@ -140,7 +140,7 @@ __device__ __forceinline__ void accelerations_with(const float* th, const float*
       const float ap0 = aw;
       const float ap1 = (c * ax + s * xy) + c1;
       const float ap2 = ((-s) * ax + c * xy) + c2;
-      const float qdd = div(uu[i] - ((U0[i] * ap0 + U1[i] * ap1) + U2[i] * ap2), U0[i], recip(U0[i]));
+      const float qdd = div(uu[i] - ((U0[i] * ap0 + U1[i] * ap1) + U2[i] * ap2), U0[i], recip_normal(U0[i]));
       aw = ap0 + qdd;
       ax = ap1;
       ay = ap2;
@@ -214,8 +214,7 @@ __device__ __forceinline__ void mass_matrix_accelerations_with(const float* th, 
 #pragma unroll
       for (int p = 0; p < j; ++p) t = t - L[i][p] * L[j][p];
       if (i == j) {
-        L[i][i] = sqrt_rn(t);
-        rL[i] = recip(L[i][i]);
+        L[i][i] = sqrt_pivot(t, &rL[i]);
       } else {
         L[i][j] = div(t, L[j][j], rL[j]);
       }
@@ -507,7 +506,7 @@ __device__ __forceinline__ void staged_inward(const float (&vw)[K], const float 
       sv[i - kStageLinks] = sn_l[(i - kStageLinks) * kBlock];
     }
     const float D = A0;
-    const double rD = recip(D);
+    const double rD = recip_normal(D);  // D >= 1: a link's own inertia plus what it carries
     const float I0 = A0 - div(A0 * A0, D, rD), I1 = A1 - div(A0 * A1, D, rD), I2 = A2 - div(A0 * A2, D, rD);
     const float I3 = A3 - div(A1 * A1, D, rD), I4 = A4 - div(A1 * A2, D, rD), I5 = A5 - div(A2 * A2, D, rD);
     const float c1 = qdv[i] * vy[i], c2 = (-qdv[i]) * vx[i];
@@ -736,7 +735,7 @@ __device__ __forceinline__ void rk4_inward(const float (&vw)[K], const float (&v
       sv[i - kStageLinks] = sn_l[(i - kStageLinks) * kBlock];
     }
     const float D = A0;
-    const double rD = recip(D);
+    const double rD = recip_normal(D);  // D >= 1: a link's own inertia plus what it carries
     const float I0 = A0 - div(A0 * A0, D, rD), I1 = A1 - div(A0 * A1, D, rD), I2 = A2 - div(A0 * A2, D, rD);
     const float I3 = A3 - div(A1 * A1, D, rD), I4 = A4 - div(A1 * A2, D, rD), I5 = A5 - div(A2 * A2, D, rD);
     const float qd = o[i] - o[i - 1];

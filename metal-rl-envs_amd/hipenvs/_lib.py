@@ -38,6 +38,7 @@ SIGNATURES = {
     "hipenvs_detmath": [_P, _P, _P, _P, _I64, _P],
     "hipenvs_div_recip": [_P, _P, _P, _P, _I64, _P],
     "hipenvs_sqrt_recip_check": [_U64, _U64, _P, _P],
+    "hipenvs_arith_check": [_U64, _U64, _P, _P],
     "hipenvs_cartpole_es_rollout": [_P, _P, _I64, _I32, _I32, _P, _P],
     "hipenvs_acrobot_reset": [_P, _I64, _U32, _P],
     "hipenvs_acrobot_step": [_P, _P, _U32, _P, _P, _P, _I64, _P],

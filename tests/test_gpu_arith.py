@@ -87,3 +87,15 @@ def test_sqrt_recip_check_argument_bounds(dev):
     _lib.call("hipenvs_sqrt_recip_check", 0, 0, _lib.ptr(counts), _lib.stream_of(dev))
     assert counts.cpu().tolist() == [0, 0]
 
+
+@pytest.mark.gpu
+def test_shortened_arithmetic_matches_the_plain_forms_for_every_float32(dev):
+    """det_tanh (fused exact products, reciprocal-estimate quotient), the fused sin/cos argument
+    reduction, the Cholesky pivots' square root, and the third-order float64 reciprocals, over
+    all 2^32 float32 bit patterns. The first three are exact by bits; the reciprocals feed one
+    rounded float64 product, which is the IEEE quotient while they are within 2^-50."""
+    counts = torch.zeros(4, dtype=torch.int64, device=dev)
+    step = 1 << 28
+    for first in range(0, 1 << 32, step):
+        _lib.call("hipenvs_arith_check", first, step, _lib.ptr(counts), _lib.stream_of(dev))
+    assert counts.cpu().tolist() == [0, 0, 0, 0]
