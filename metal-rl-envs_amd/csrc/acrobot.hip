@@ -9,7 +9,7 @@
 // counter RNG of acrobot_metal.py:78-83. Per env-step the step kernel moves 41
 // algorithmic bytes; it is VALU-bound (14 sin/cos, 18 IEEE divisions).
 
-#include "es_noise.h"
+#include "es_rollout.h"
 
 namespace hipenvs {
 namespace ac {
@@ -33,9 +33,7 @@ constexpr float MAX_VEL_1 = 0x1.921fb6p+3f;   // float32(4 * pi)
 constexpr float MAX_VEL_2 = 0x1.c463acp+4f;   // float32(9 * pi)
 constexpr float RESET_BOUND = 0x1.99999ap-4f; // float32(0.1)
 
-struct S4 {
-  float a, b, c, d;  // theta1, theta2, dtheta1, dtheta2 (or their derivatives)
-};
+using S4 = roll::State4;  // theta1, theta2, dtheta1, dtheta2 (or their derivatives)
 
 // acrobot_np.py:64-84. The numpy expression's multiplications by the Python
 // float 1.0 (m2 *, 2 * l1 * lc2 *) are exact and omitted.
@@ -126,59 +124,6 @@ __global__ __launch_bounds__(kBlock) void step_kernel(const float* __restrict__ 
   stream_store((uint8_t)(d ? 1 : 0), done + i);
 }
 
-// Fused ES rollout: one thread per member, the member's 10H+3 weights in
-// registers (es.unflatten layout: w1 (6, H), b1 (H), w2 (H, 3), b2 (3)),
-// Gym's observation, first-index argmax over three torques, RK4 physics, stop
-// at the first termination. acrobot_rollout_metal.py:21-58.
-template <int H>
-__global__ __launch_bounds__(64) void rollout_kernel(const float* __restrict__ state, const float* __restrict__ theta,
-                                                     int64_t member_stride, int64_t p, int32_t horizon,
-                                                     float out_sign, float* __restrict__ steps_out) {
-  constexpr int D = 10 * H + 3;
-  const int64_t i = (int64_t)blockIdx.x * 64 + threadIdx.x;
-  if (i >= p) return;
-  const float* row = theta + i * member_stride;
-  float w[D];
-#pragma unroll
-  for (int d = 0; d < D; ++d) w[d] = row[d];
-  S4 s{state[i], state[p + i], state[2 * p + i], state[3 * p + i]};
-  float steps = 0.0f;
-  for (int32_t t = 0; t < horizon; ++t) {
-    float o[6];
-    det_sincos(s.a, &o[1], &o[0]);
-    det_sincos(s.b, &o[3], &o[2]);
-    o[4] = s.c;
-    o[5] = s.d;
-    float l0 = w[10 * H], l1 = w[10 * H + 1], l2 = w[10 * H + 2];
-#pragma unroll
-    for (int j = 0; j < H; ++j) {
-      float pre = o[0] * w[j];
-#pragma unroll
-      for (int k = 1; k < 6; ++k) pre = pre + o[k] * w[k * H + j];
-      const float h = det_tanh(pre + w[6 * H + j]);
-      l0 = l0 + h * w[7 * H + 3 * j];
-      l1 = l1 + h * w[7 * H + 3 * j + 1];
-      l2 = l2 + h * w[7 * H + 3 * j + 2];
-    }
-    float torque = -1.0f, best = l0;
-    if (l1 > best) { torque = 0.0f; best = l1; }
-    if (l2 > best) { torque = 1.0f; }
-    rk4(s, torque);
-    if (terminal(s)) break;
-    steps += 1.0f;
-  }
-  steps_out[i] = out_sign * steps + 0.0f;  // + 0: a score of -0 reads +0
-}
-
-// The same rollout with a group of kRolloutLanes lanes per member (four members to a
-// single-wave workgroup), for populations that would fill only a fraction of the SIMDs with
-// one member per lane: lane g computes hidden units g, g + 16, ... from the weights it holds;
-// lanes 0..2 sum the three heads over all hidden values, read in order from the group's LDS
-// row; observation and RK4 physics run identically on all 16 lanes. Same bits as the one-lane
-// form.
-constexpr int kRolloutLanes = 16;
-constexpr int kRolloutMembers = 64 / kRolloutLanes;
-
 // The group's physics, with the transcendentals and the two quotients by d1 spread over the
 // group's lanes: lanes 0, 1, 2 evaluate one det_sincos each (one instruction stream for the
 // three) and every lane of the 16-lane group (one DPP row) receives the results by row
@@ -188,39 +133,42 @@ struct GroupTrig {
   float sin_a, cos_a, sin_b, cos_b, cos_ab;  // theta1, theta2, theta2 + theta1
 };
 
+template <int G>
 __device__ __forceinline__ GroupTrig group_trig(const S4& s, int g) {
   const float x = (g == 1) ? s.b : (g == 2) ? (s.b + s.a) : s.a;
   float sn, cs;
   det_sincos(x, &sn, &cs);
-  return GroupTrig{group_bcast<0>(sn), group_bcast<0>(cs), group_bcast<1>(sn), group_bcast<1>(cs),
-                   group_bcast<2>(cs)};
+  return GroupTrig{lane_bcast<G, 0>(sn), lane_bcast<G, 0>(cs), lane_bcast<G, 1>(sn), lane_bcast<G, 1>(cs),
+                   lane_bcast<G, 2>(cs)};
 }
 
+template <int G>
 __device__ __forceinline__ S4 dsdt_group(const S4& s, float torque, int g) {
   const float x = (g == 1) ? ((s.a + s.b) - HALF_PI) : (g == 2) ? (s.a - HALF_PI) : s.b;
   float sn, cs;
   det_sincos(x, &sn, &cs);
-  const float s2 = group_bcast<0>(sn), c2 = group_bcast<0>(cs);
+  const float s2 = lane_bcast<G, 0>(sn), c2 = lane_bcast<G, 0>(cs);
   const float d1 = ((D1_C0 + (D1_C1 + c2)) + 1.0f) + 1.0f;
   const float d2 = (D2_C0 + D2_C1 * c2) + 1.0f;
-  const float phi2 = PHI2_C * group_bcast<1>(cs);
+  const float phi2 = PHI2_C * lane_bcast<G, 1>(cs);
   const float t1 = (PHI1_A * (s.d * s.d)) * s2;
   const float t2 = (s.d * s.c) * s2;
-  const float t3 = PHI1_C * group_bcast<2>(cs);
+  const float t3 = PHI1_C * lane_bcast<G, 2>(cs);
   const float phi1 = ((t1 - t2) + t3) + phi2;
   const float q = ((g == 1) ? d2 * d2 : d2) / d1;  // lane 0: d2 / d1, lane 1: (d2 * d2) / d1
-  const float num = ((torque + group_bcast<0>(q) * phi1) - (DD2_C * (s.c * s.c)) * s2) - phi2;
-  const float den = DEN_C - group_bcast<1>(q);
+  const float num = ((torque + lane_bcast<G, 0>(q) * phi1) - (DD2_C * (s.c * s.c)) * s2) - phi2;
+  const float den = DEN_C - lane_bcast<G, 1>(q);
   const float dd2 = num / den;
   const float dd1 = (-((d2 * dd2) + phi1)) / d1;
   return S4{s.c, s.d, dd1, dd2};
 }
 
+template <int G>
 __device__ __forceinline__ void rk4_group(S4& s, float torque, int g) {
-  const S4 k1 = dsdt_group(s, torque, g);
-  const S4 k2 = dsdt_group(S4{s.a + DT_2 * k1.a, s.b + DT_2 * k1.b, s.c + DT_2 * k1.c, s.d + DT_2 * k1.d}, torque, g);
-  const S4 k3 = dsdt_group(S4{s.a + DT_2 * k2.a, s.b + DT_2 * k2.b, s.c + DT_2 * k2.c, s.d + DT_2 * k2.d}, torque, g);
-  const S4 k4 = dsdt_group(S4{s.a + DT * k3.a, s.b + DT * k3.b, s.c + DT * k3.c, s.d + DT * k3.d}, torque, g);
+  const S4 k1 = dsdt_group<G>(s, torque, g);
+  const S4 k2 = dsdt_group<G>(S4{s.a + DT_2 * k1.a, s.b + DT_2 * k1.b, s.c + DT_2 * k1.c, s.d + DT_2 * k1.d}, torque, g);
+  const S4 k3 = dsdt_group<G>(S4{s.a + DT_2 * k2.a, s.b + DT_2 * k2.b, s.c + DT_2 * k2.c, s.d + DT_2 * k2.d}, torque, g);
+  const S4 k4 = dsdt_group<G>(S4{s.a + DT * k3.a, s.b + DT * k3.b, s.c + DT * k3.c, s.d + DT * k3.d}, torque, g);
   const float na = s.a + DT_6 * (((k1.a + 2.0f * k2.a) + 2.0f * k3.a) + k4.a);
   const float nb = s.b + DT_6 * (((k1.b + 2.0f * k2.b) + 2.0f * k3.b) + k4.b);
   const float nc = s.c + DT_6 * (((k1.c + 2.0f * k2.c) + 2.0f * k3.c) + k4.c);
@@ -231,105 +179,73 @@ __device__ __forceinline__ void rk4_group(S4& s, float torque, int g) {
   s.d = clip(nd, -MAX_VEL_2, MAX_VEL_2);
 }
 
-template <int H>
-__global__ __launch_bounds__(64) void rollout_group_kernel(const float* __restrict__ state,
-                                                           const float* __restrict__ theta, int64_t member_stride,
-                                                           int64_t p, int32_t horizon, float out_sign,
-                                                           float* __restrict__ steps_out) {
-  constexpr int G = kRolloutLanes, U = (H + G - 1) / G;
-  __shared__ float xp_all[kRolloutMembers * 3 * H];
-  __shared__ float xl_all[kRolloutMembers * 4];
-  const int g = (int)threadIdx.x % G, mloc = (int)threadIdx.x / G;
-  float* xp = xp_all + mloc * 3 * H;  // head o's terms h_j * w2[j][o] at o * H + j
-  float* xl = xl_all + mloc * 4;
-  const int64_t i = (int64_t)blockIdx.x * kRolloutMembers + mloc;
-  bool alive = i < p;
-  const int64_t m = alive ? i : p - 1;  // a group past p steps member p - 1, unused
-  const float* row = theta + m * member_stride;
-  float w1[U][6], b1[U], w2[U][3];
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int j = g + G * u < H ? g + G * u : 0;  // lanes past H recompute unit 0, unused
-#pragma unroll
-    for (int k = 0; k < 6; ++k) w1[u][k] = row[k * H + j];
-    b1[u] = row[6 * H + j];
-#pragma unroll
-    for (int oo = 0; oo < 3; ++oo) w2[u][oo] = row[7 * H + 3 * j + oo];
-  }
-  const int o = g < 3 ? g : 0;
-  const float b2 = row[10 * H + o];
-  const float* xo = xp + o * H;
-  S4 s{state[m], state[p + m], state[2 * p + m], state[3 * p + m]};
-  float steps = 0.0f;
-  int32_t t = 0;
-  alive = alive && horizon > 0;
-  GroupTrig tr = group_trig(s, g);  // the observation's trig; after each step also the termination's
-  while (__any(alive)) {  // every lane steps, so the barriers and row broadcasts stay uniform
-    float ob[6];
-    ob[0] = tr.cos_a;
-    ob[1] = tr.sin_a;
-    ob[2] = tr.cos_b;
-    ob[3] = tr.sin_b;
-    ob[4] = s.c;
-    ob[5] = s.d;
-    // each lane forms its units' head terms h_j * w2[j][o], and lanes 0-2 add them in
-    // order: the same products and sums as one lane summing l + h_j * w2[j][o], with the
-    // multiplications spread over the group instead of repeated on the head lanes
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      float pre = ob[0] * w1[u][0];
-#pragma unroll
-      for (int k = 1; k < 6; ++k) pre = pre + ob[k] * w1[u][k];
-      const float h = det_tanh(pre + b1[u]);
-      if (g + G * u < H) {
-#pragma unroll
-        for (int oo = 0; oo < 3; ++oo) xp[oo * H + g + G * u] = h * w2[u][oo];
-      }
-    }
-    __syncthreads();
-    if (g < 3) {
-      float l = b2;
-#pragma unroll
-      for (int j = 0; j < H; ++j) l = l + xo[j];
-      xl[g] = l;
-    }
-    __syncthreads();
-    const float l0 = xl[0], l1 = xl[1], l2 = xl[2];
-    __syncthreads();  // the group's rows are read before the next step writes them
-    float torque = -1.0f, best = l0;
-    if (l1 > best) { torque = 0.0f; best = l1; }
-    if (l2 > best) { torque = 1.0f; }
-    rk4_group(s, torque, g);
-    tr = group_trig(s, g);
-    const bool done = (-tr.cos_a) - tr.cos_ab > 1.0f;  // terminal(s)
-    if (alive) {
-      if (done) {
-        alive = false;
-      } else {
-        steps += 1.0f;
-        alive = ++t < horizon;
-      }
+// The fused ES rollout's body (es_rollout.h): Gym's observation, the 6-H-3 tanh policy with
+// first-index argmax over three torques, RK4 physics, stop at the first termination
+// (acrobot_rollout_metal.py:21-58). A population's score is the steps survived (sign 1), the
+// greedy evaluation's minus the steps (sign -1).
+struct RolloutBody {
+  static constexpr int kIn = 6, kOut = 3;
+  template <int H, int G>
+  static constexpr int kMinWaves = 1;
+  using Trig = GroupTrig;  // the observation's trig; after each step also the termination's
+  template <int G>
+  __device__ static __forceinline__ Trig trig(const S4& s, int g) {
+    if constexpr (G == 1) {
+      Trig t;
+      det_sincos(s.a, &t.sin_a, &t.cos_a);
+      det_sincos(s.b, &t.sin_b, &t.cos_b);
+      t.cos_ab = det_cos(s.b + s.a);
+      return t;
+    } else {
+      return group_trig<G>(s, g);
     }
   }
-  if (g == 0 && i < p) steps_out[i] = out_sign * steps + 0.0f;  // + 0: a score of -0 reads +0
-}
+  __device__ static __forceinline__ void observe(const S4& s, const Trig& t, float (&obs)[6]) {
+    obs[0] = t.cos_a;
+    obs[1] = t.sin_a;
+    obs[2] = t.cos_b;
+    obs[3] = t.sin_b;
+    obs[4] = s.c;
+    obs[5] = s.d;
+  }
+  template <int G>
+  __device__ static __forceinline__ bool step(S4& s, Trig& t, const float (&l)[3], bool, int g) {
+    float torque = -1.0f, best = l[0];
+    if (l[1] > best) { torque = 0.0f; best = l[1]; }
+    if (l[2] > best) { torque = 1.0f; }
+    if constexpr (G == 1)
+      rk4(s, torque);
+    else
+      rk4_group<G>(s, torque, g);
+    t = trig<G>(s, g);
+    return (-t.cos_a) - t.cos_ab > 1.0f;  // terminal(s)
+  }
+  // steps as a float32 count that stops at 2^24, where adding one no longer changes it; + 0: a
+  // score of -0 reads +0
+  __device__ static __forceinline__ float score(int32_t t, float sign) {
+    return sign * (float)(t < 0x1000000 ? t : 0x1000000) + 0.0f;
+  }
+};
 
-// member_stride D and out_sign 1 for a population's rollout; stride 0 (one shared policy)
-// and sign -1 for the greedy evaluation, whose per-env score is minus the steps.
+// Lanes per member at the start, by members per CU (500 steps, most members run them all; P
+// on 256 CUs, us; 16 / 4 / 1 lanes):
+//   H = 32: P = 4,096 826 / 1,074 / 2,455; 8,192 1,262 / 1,128 / 2,464; 32,768 4,594 / 1,973 /
+//           2,507; 65,536 8,044 / 2,960 / 2,503; 262,144 29,660 / 10,715 / 9,938
+//   H = 8:  P = 4,096 795 / 778 / 1,305; 32,768 3,619 / 1,141 / 1,330; 65,536 6,849 / 2,148 / 1,317
+//   H = 64: P = 32,768 5,694 / 2,319, one lane 5,108; 262,144 16,475, one lane 26,696
+constexpr int kGroup16PerCu = 16, kGroup4PerCu = 128;
+
 template <int H>
 int launch_rollout(const float* state, const float* theta, int64_t member_stride, int64_t p, int32_t horizon,
-                   float out_sign, float* out, hipStream_t s) {
-  int64_t limit = 0;
-  const int status = group_rollout_limit(&limit);
+                   float sign, float* out, hipStream_t s) {
+  int cus = 0;
+  const int status = device_cus(&cus);
   if (status != HIPENVS_OK) return status;
-  if (p <= limit) {
-    hipLaunchKernelGGL(rollout_group_kernel<H>, dim3((unsigned)((p + kRolloutMembers - 1) / kRolloutMembers)),
-                       dim3(64), 0, s, state, theta, member_stride, p, horizon, out_sign, out);
-  } else {
-    hipLaunchKernelGGL(rollout_kernel<H>, dim3(grid_for(p, 64)), dim3(64), 0, s, state, theta, member_stride, p,
-                       horizon, out_sign, out);
-  }
-  return launch_status();
+  if (p <= (int64_t)kGroup16PerCu * cus)
+    return roll::launch<RolloutBody, H, 16>(state, theta, member_stride, p, horizon, sign, out, s);
+  if (H > 32 || p <= (int64_t)kGroup4PerCu * cus)
+    return roll::launch<RolloutBody, H, 4>(state, theta, member_stride, p, horizon, sign, out, s);
+  return roll::launch<RolloutBody, H, (H > 32 ? 4 : 1)>(state, theta, member_stride, p, horizon, sign, out, s);
 }
 
 template <int H>

@@ -9,7 +9,7 @@
 // moves 41 algorithmic bytes: 16 B state in, 4 B action, 16 B state out,
 // 4 B reward, 1 B done.
 
-#include "es_noise.h"
+#include "es_rollout.h"
 
 namespace hipenvs {
 namespace cp {
@@ -133,133 +133,60 @@ __global__ __launch_bounds__(kBlock) void sample_actions_kernel(int32_t* __restr
   action[i] = (m == 2u) ? action_bit(h) : action_uniform(h, m);
 }
 
-// Fused ES rollout: one thread per member, the member's 7H+2 weights in
-// registers (es.unflatten layout: w1 (4, H), b1 (H), w2 (H, 2), b2 (2)), the
-// 4-H-2 tanh policy with first-index argmax, the step physics, and an early
-// exit at the first termination; writes the steps survived (the terminating
-// step not counted). cartpole_rollout_metal.py:46-77. Member i's weights start
-// at theta + i * member_stride: D for a population, 0 for one policy shared by
-// every env (the greedy evaluation).
-template <int H>
-__global__ __launch_bounds__(64) void rollout_kernel(const float* __restrict__ state, const float* __restrict__ theta,
-                                                     int64_t member_stride, int64_t p, int32_t horizon,
-                                                     float* __restrict__ fitness) {
-  const int64_t i = (int64_t)blockIdx.x * 64 + threadIdx.x;
-  if (i >= p) return;
-  constexpr int D = 7 * H + 2;
-  const float* row = theta + i * member_stride;
-  float w[D];
-#pragma unroll
-  for (int d = 0; d < D; ++d) w[d] = row[d];
-  float x = state[i], xd = state[p + i], th = state[2 * p + i], thd = state[3 * p + i];
-  float survived = 0.0f;
-  for (int32_t t = 0; t < horizon; ++t) {
-    float l0 = w[7 * H], l1 = w[7 * H + 1];
-#pragma unroll
-    for (int j = 0; j < H; ++j) {
-      const float pre = (((x * w[j] + xd * w[H + j]) + th * w[2 * H + j]) + thd * w[3 * H + j]) + w[4 * H + j];
-      const float h = det_tanh(pre);
-      l0 = l0 + h * w[5 * H + 2 * j];
-      l1 = l1 + h * w[5 * H + 2 * j + 1];
-    }
-    if (advance(x, xd, th, thd, (l1 > l0) ? 1 : 0)) break;
-    survived += 1.0f;
+// The fused ES rollout's body (es_rollout.h): the 4-H-2 tanh policy with first-index argmax and
+// the step physics; a member's score is the steps survived, the terminating step not counted
+// (cartpole_rollout_metal.py:46-77).
+struct RolloutBody {
+  static constexpr int kIn = 4, kOut = 2;
+  // the one-lane form keeps all 7H + 2 weights in registers: two waves per SIMD at H = 32
+  template <int H, int G>
+  static constexpr int kMinWaves = (G == 1 && H == 32) ? 2 : 1;
+  struct Trig {};
+  template <int G>
+  __device__ static __forceinline__ Trig trig(const roll::State4&, int) {
+    return {};
   }
-  fitness[i] = survived;
-}
+  __device__ static __forceinline__ void observe(const roll::State4& s, const Trig&, float (&obs)[4]) {
+    obs[0] = s.a;
+    obs[1] = s.b;
+    obs[2] = s.c;
+    obs[3] = s.d;
+  }
+  // every member steps (no branch around the physics); the near-zero sin/cos vote counts the
+  // live members alone, since a finished member's results are discarded
+  template <int G>
+  __device__ static __forceinline__ bool step(roll::State4& s, Trig&, const float (&l)[2], bool alive, int) {
+    return advance(s.a, s.b, s.c, s.d, (l[1] > l[0]) ? 1 : 0, alive);
+  }
+  // steps as a float32 count that stops at 2^24, where adding one no longer changes it
+  __device__ static __forceinline__ float score(int32_t t, float) { return (float)(t < 0x1000000 ? t : 0x1000000); }
+};
 
-// The same rollout with a group of kRolloutLanes lanes per member (four members to a
-// single-wave workgroup), for populations that would fill only a fraction of the SIMDs with
-// one member per lane: lane g computes hidden units g, g + 16, ... from the weights it holds;
-// lanes 0 and 1 sum the two heads over all hidden values, read in order from the group's LDS
-// row; the physics runs identically on all 16 lanes. A member's step then costs about a
-// quarter of the one-lane form's instruction latency, and the results are the same bits.
-constexpr int kRolloutLanes = 16;
-constexpr int kRolloutMembers = 64 / kRolloutLanes;
-
+// Lanes per member at the start, by members per CU. Trained populations (every member runs
+// the 500 steps, P on 256 CUs, us; 16 / 4 / 1 lanes):
+//   H = 32: P = 4,096 293 / 489 / 1,379; 8,192 356 / 530 / 1,383; 32,768 1,002 / 819 / 1,413;
+//           65,536 1,816 / 1,294 / 1,416; 262,144 6,689 / 4,387 / 4,133
+//   H = 8:  P = 8,192 240 / 264 / 446; 32,768 631 / 296 / 469; 65,536 1,089 / 456 / 449
+//   H = 64: P = 8,192 563 / 916; 65,536 3,153 / 2,378 (its 450 weights leave one lane one wave
+//           per SIMD: 2,864)
+// Populations early in training, whose waves narrow as their members fail, are within 10 %
+// between the forms at these bounds. (One member per lane to the end, as before: P = 262,144,
+// H = 32 early in training 2,844 us, now 402; trained 5,147, now 4,133.)
+constexpr int kGroup16PerCu = 32;
 template <int H>
-__global__ __launch_bounds__(64) void rollout_group_kernel(const float* __restrict__ state,
-                                                           const float* __restrict__ theta, int64_t member_stride,
-                                                           int64_t p, int32_t horizon, float* __restrict__ fitness) {
-  constexpr int G = kRolloutLanes, U = (H + G - 1) / G;
-  __shared__ float xp_all[kRolloutMembers * 2 * H];
-  __shared__ float xl_all[kRolloutMembers * 2];
-  const int g = (int)threadIdx.x % G, mloc = (int)threadIdx.x / G;
-  float* xp = xp_all + mloc * 2 * H;  // head o's terms h_j * w2[j][o] at o * H + j
-  float* xl = xl_all + mloc * 2;
-  const int64_t i = (int64_t)blockIdx.x * kRolloutMembers + mloc;
-  bool alive = i < p;
-  const int64_t m = alive ? i : p - 1;  // a group past p steps member p - 1, unused
-  const float* row = theta + m * member_stride;
-  float w1[U][4], b1[U], w2[U][2];
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int j = g + G * u < H ? g + G * u : 0;  // lanes past H recompute unit 0, unused
-#pragma unroll
-    for (int k = 0; k < 4; ++k) w1[u][k] = row[k * H + j];
-    b1[u] = row[4 * H + j];
-    w2[u][0] = row[5 * H + 2 * j];
-    w2[u][1] = row[5 * H + 2 * j + 1];
-  }
-  const int o = g < 2 ? g : 0;
-  const float b2 = row[7 * H + o];
-  const float* xo = xp + o * H;
-  float x = state[m], xd = state[p + m], th = state[2 * p + m], thd = state[3 * p + m];
-  float survived = 0.0f;
-  int32_t t = 0;
-  alive = alive && horizon > 0;
-  while (__any(alive)) {  // every lane steps, so the barriers stay uniform
-    // each lane forms its units' head terms h_j * w2[j][o], and lanes 0 and 1 add them in
-    // order: the same products and sums as one lane summing l + h_j * w2[j][o], with the
-    // multiplications spread over the group instead of repeated on the head lanes
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const float pre = (((x * w1[u][0] + xd * w1[u][1]) + th * w1[u][2]) + thd * w1[u][3]) + b1[u];
-      const float h = det_tanh(pre);
-      if (g + G * u < H) {
-        xp[g + G * u] = h * w2[u][0];
-        xp[H + g + G * u] = h * w2[u][1];
-      }
-    }
-    __syncthreads();
-    if (g < 2) {
-      float l = b2;
-#pragma unroll
-      for (int j = 0; j < H; ++j) l = l + xo[j];
-      xl[g] = l;
-    }
-    __syncthreads();
-    const float l0 = xl[0], l1 = xl[1];
-    __syncthreads();  // the group's rows are read before the next step writes them
-    // every member steps (no branch around the physics); the near-zero sin/cos vote counts
-    // the live members alone, since a terminated member's results are discarded
-    const bool done = advance(x, xd, th, thd, (l1 > l0) ? 1 : 0, alive);
-    if (alive) {
-      if (done) {
-        alive = false;
-      } else {
-        survived += 1.0f;
-        alive = ++t < horizon;
-      }
-    }
-  }
-  if (g == 0 && i < p) fitness[i] = survived;
-}
+constexpr int kGroup4PerCu = H >= 16 ? 256 : 128;
 
 template <int H>
 int launch_rollout(const float* state, const float* theta, int64_t member_stride, int64_t p, int32_t horizon,
                    float* out, hipStream_t s) {
-  int64_t limit = 0;
-  const int status = group_rollout_limit(&limit);
+  int cus = 0;
+  const int status = device_cus(&cus);
   if (status != HIPENVS_OK) return status;
-  if (p <= limit) {
-    hipLaunchKernelGGL(rollout_group_kernel<H>, dim3((unsigned)((p + kRolloutMembers - 1) / kRolloutMembers)),
-                       dim3(64), 0, s, state, theta, member_stride, p, horizon, out);
-  } else {
-    hipLaunchKernelGGL(rollout_kernel<H>, dim3(grid_for(p, 64)), dim3(64), 0, s, state, theta, member_stride, p,
-                       horizon, out);
-  }
-  return launch_status();
+  if (p <= (int64_t)kGroup16PerCu * cus)
+    return roll::launch<RolloutBody, H, 16>(state, theta, member_stride, p, horizon, 1.0f, out, s);
+  if (H > 32 || p <= (int64_t)kGroup4PerCu<H> * cus)
+    return roll::launch<RolloutBody, H, 4>(state, theta, member_stride, p, horizon, 1.0f, out, s);
+  return roll::launch<RolloutBody, H, (H > 32 ? 4 : 1)>(state, theta, member_stride, p, horizon, 1.0f, out, s);
 }
 
 template <int H>

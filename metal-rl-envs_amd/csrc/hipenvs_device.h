@@ -115,12 +115,23 @@ __device__ __forceinline__ void sincos_quadrant(float r, int q, float* sin_out, 
   *cos_out = ((q + 1) & 2) ? -b : b;
 }
 
+// kFused false keeps the reduction's plain form, for kernels out of registers (with the fused
+// one the K = 64 RK4 pendulum spilled 276 instead of 212 B/lane: 182.8 against 180.5 us).
+template <bool kFused = true>
 __device__ __forceinline__ void det_sincos(float x, float* sin_out, float* cos_out) {
   // float32 reduction, computed for every lane on an argument clamped into its range (so
   // no branch precedes it and independent work can overlap the loads that feed x) ...
   const bool small = fabsf(x) <= dm::SMALL_ARG;
+  const float xs = small ? x : 0.0f;
   int q;
-  float r = reduce_small(small ? x : 0.0f, &q);
+  float r;
+  if constexpr (kFused) {
+    r = reduce_small(xs, &q);
+  } else {
+    const float k = rintf(xs * dm::TWO_OVER_PI);
+    r = (((xs - k * dm::PIO2_1) - k * dm::PIO2_2) - k * dm::PIO2_3) - k * dm::PIO2_4;
+    q = (int)k & 3;
+  }
   if (!small) {  // ... and the float64 reduction for |x| > 256, inf and NaN
     const double xd = (double)x;
     const double kd = rint(xd * dm::TWO_OVER_PI_D);
@@ -131,6 +142,10 @@ __device__ __forceinline__ void det_sincos(float x, float* sin_out, float* cos_o
   sincos_quadrant(r, q, sin_out, cos_out);
 }
 
+// Whether `p` holds on every active lane (HIP's __all goes through an integer per lane: a
+// select, a compare and two scalar instructions more).
+__device__ __forceinline__ bool wave_all(bool p) { return __builtin_amdgcn_ballot_w64(!p) == 0ull; }
+
 // det_sincos of K arguments under one wave vote: when every active lane has all K of them
 // within 256 (always, for wrapped angles) the float32 reductions alone, with no branch
 // between them, so the K streams interleave; det_sincos of each otherwise.
@@ -139,7 +154,7 @@ __device__ __forceinline__ void det_sincos_small(const float (&x)[K], float (&si
   bool ok = true;
 #pragma unroll
   for (int i = 0; i < K; ++i) ok &= fabsf(x[i]) <= dm::SMALL_ARG;
-  if (__all(ok)) {
+  if (wave_all(ok)) {
 #pragma unroll
     for (int i = 0; i < K; ++i) {
       int q;
@@ -197,6 +212,8 @@ __device__ __forceinline__ void det_sincos64(double x, double* sin_out, double* 
 // Lanes with `counts` false take no part in the vote, and their results are not det_sincos's
 // when the wave takes the polynomial: for callers that discard those lanes' results.
 __device__ __forceinline__ void det_sincos_near_zero(float x, float* sin_out, float* cos_out, bool counts = true) {
+  // HIP's __all here: with wave_all the compiler lays the rare path out first, and the K-step
+  // kernel took 71.3 instead of 69.6 us at N = 2^20
   if (__all(!counts || fabsf(x) <= 0.78f)) {
     sincos_poly(x, sin_out, cos_out);
   } else {
@@ -213,7 +230,7 @@ __device__ __forceinline__ bool wave_near_zero(const float* x) {
   bool ok = true;
 #pragma unroll
   for (int i = 0; i < K; ++i) ok &= fabsf(x[i]) <= 0.78f;
-  return __all(ok);
+  return wave_all(ok);
 }
 
 // det_sincos of K arguments; the polynomial alone when the wave's vote allows it.
@@ -271,9 +288,10 @@ __device__ __forceinline__ float det_sin(float x) {
   return s;
 }
 
+template <bool kFused = true>
 __device__ __forceinline__ float det_cos(float x) {
   float s, c;
-  det_sincos(x, &s, &c);
+  det_sincos<kFused>(x, &s, &c);
   return c;
 }
 
@@ -287,27 +305,52 @@ __device__ __forceinline__ float det_cos(float x) {
 //   the separate ones do;
 // - e / (e + 2) from the reciprocal estimate and one residual correction, equal to the IEEE
 //   quotient for each of the 2^32 inputs (hipenvs_arith_check, run by the GPU tests).
-__device__ __forceinline__ float det_tanh(float x) {
+// det_tanh_all<N> forms N of them a step at a time: a tanh is one dependent chain, and the
+// compiler otherwise finishes one before it starts the next.
+template <int N>
+__device__ __forceinline__ void det_tanh_all(const float (&x)[N], float (&out)[N]) {
   constexpr float kRound = 0x1.8p+23f;
-  float a = fabsf(x);
-  a = (a > dm::TANH_CLAMP) ? dm::TANH_CLAMP : a;  // NaN compares false and stays NaN
-  const float y = a + a;
-  const float t = y * dm::LOG2E + kRound;
-  const float k = t - kRound;
-  const float r = __builtin_fmaf(-k, dm::LN2_HI, y) - k * dm::LN2_LO;
-  float p = dm::E7 + r * dm::E8;
-  p = dm::E6 + r * p;
-  p = dm::E5 + r * p;
-  p = dm::E4 + r * p;
-  p = dm::E3 + r * p;
-  p = dm::E2 + r * p;
-  p = r + (r * r) * p;
-  const float two_k = __uint_as_float((__float_as_uint(t) << 23) + 0x3F800000u);
-  const float e = __builtin_fmaf(two_k, p, two_k - 1.0f);
-  const float d = e + 2.0f;
-  const float rd = __builtin_amdgcn_rcpf(d);
-  const float q = e * rd;
-  return copysignf(__builtin_fmaf(__builtin_fmaf(-q, d, e), rd, q), x);
+  constexpr float kPoly[7] = {dm::E8, dm::E7, dm::E6, dm::E5, dm::E4, dm::E3, dm::E2};
+  float y[N], t[N], r[N], p[N], e[N], rd[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    float a = fabsf(x[i]);
+    a = (a > dm::TANH_CLAMP) ? dm::TANH_CLAMP : a;  // NaN compares false and stays NaN
+    y[i] = a + a;
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) t[i] = y[i] * dm::LOG2E + kRound;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const float k = t[i] - kRound;
+    r[i] = __builtin_fmaf(-k, dm::LN2_HI, y[i]) - k * dm::LN2_LO;
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) p[i] = kPoly[0];
+#pragma unroll
+  for (int c = 1; c < 7; ++c)
+#pragma unroll
+    for (int i = 0; i < N; ++i) p[i] = kPoly[c] + r[i] * p[i];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    p[i] = r[i] + (r[i] * r[i]) * p[i];
+    const float two_k = __uint_as_float((__float_as_uint(t[i]) << 23) + 0x3F800000u);
+    e[i] = __builtin_fmaf(two_k, p[i], two_k - 1.0f);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) rd[i] = __builtin_amdgcn_rcpf(e[i] + 2.0f);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const float q = e[i] * rd[i];
+    out[i] = copysignf(__builtin_fmaf(__builtin_fmaf(-q, e[i] + 2.0f, e[i]), rd[i], q), x[i]);
+  }
+}
+
+__device__ __forceinline__ float det_tanh(float x) {
+  const float in[1] = {x};
+  float out[1];
+  det_tanh_all<1>(in, out);
+  return out[0];
 }
 
 // x / c for a float32 constant c, as one float64 product with inv_c = 1 / (double)c
@@ -446,15 +489,6 @@ int current_device(int* dev);
 // Compute units of the current device, queried once per device (the answer cannot change
 // while the process runs); a negative status when the query fails.
 int device_cus(int* cus);
-
-// Populations up to this size run the fused ES rollouts with a lane group per member: 16
-// members per CU, i.e. one four-member wave per SIMD.
-inline int group_rollout_limit(int64_t* limit) {
-  int cus = 0;
-  const int status = device_cus(&cus);
-  *limit = 16 * (int64_t)cus;
-  return status;
-}
 
 // Resident 64-thread workgroups per CU of `kernel` on the current device, queried once per
 // device for each kernel (Tag distinguishes the callers' caches); a negative status on failure.

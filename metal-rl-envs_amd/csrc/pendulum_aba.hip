@@ -270,7 +270,7 @@ __device__ __forceinline__ bool terminal(const float* th) {
     }
   } else {
 #pragma unroll U
-    for (int i = 0; i < K; ++i) s = (i == 0) ? det_cos(th[0]) : s + det_cos(th[i]);
+    for (int i = 0; i < K; ++i) s = (i == 0) ? det_cos<(K < 64)>(th[0]) : s + det_cos<(K < 64)>(th[i]);
   }
   return -s > (float)K * 0.5f;
 }
@@ -692,7 +692,7 @@ __device__ __forceinline__ void rk4_outward(const float (&t)[K], const float (&o
     if constexpr (kNear)
       sincos_poly(q, &sn, &cs);
     else
-      det_sincos(q, &sn, &cs);
+      det_sincos<(K < 64)>(q, &sn, &cs);
     sn_l[i * kBlock] = sn;
     cs_l[i * kBlock] = cs;
     const float xy = (i == 0) ? (y + w * 0.0f) : (y + w);

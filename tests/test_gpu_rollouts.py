@@ -56,8 +56,8 @@ def test_acrobot_rollout_matches_oracle(dev, hidden):
 
 @pytest.mark.parametrize("hidden", [8, 32])
 def test_large_populations_one_member_per_lane(dev, hidden):
-    """Populations above the lane-group limit (16 members per CU) run one member per lane;
-    both bodies, bit for bit against the oracle."""
+    """Populations above the 16-lane form's bound start with fewer lanes per member; both bodies,
+    bit for bit against the oracle."""
     from hipenvs import acrobot_rollout, cartpole_rollout
 
     p = 20_000
@@ -69,6 +69,68 @@ def test_large_populations_one_member_per_lane(dev, hidden):
     state = oa.reset(p, seed=6)
     got = acrobot_rollout.rollout_steps(torch.from_numpy(state).to(dev), torch.from_numpy(theta).to(dev), hidden, 60)
     np.testing.assert_array_equal(to_np(got), oa.rollout_steps(state, theta, hidden, 60))
+
+
+def _mixed_population(body, p, hidden, seed):
+    """Half the members balance (CartPole) or are as drawn, half are wild, shuffled: a wave's
+    members fail at many different steps, so it passes through every lane-group form."""
+    i, o = (4, 2) if body == "cartpole" else (6, 3)
+    r = np.random.default_rng(seed)
+    theta = (r.standard_normal((p, i * hidden + hidden + hidden * o + o)) * 0.3).astype(np.float32)
+    if body == "cartpole":
+        good = r.random(p) < 0.5
+        theta[good] *= np.float32(0.2)
+        theta[good, :4 * hidden] += np.repeat(np.array([0.1, 0.4, 4.0, 1.2], np.float32), hidden)
+        theta[good, 5 * hidden:7 * hidden:2] -= np.float32(1.0)
+        theta[good, 5 * hidden + 1:7 * hidden:2] += np.float32(1.0)
+    return theta
+
+
+# members per CU at which the starting form changes (16, 4, 1 lanes per member), per body and H
+_FORM_BOUNDS = {("cartpole", 4): (32, 128), ("cartpole", 32): (32, 256), ("cartpole", 64): (32, None),
+                ("acrobot", 8): (16, 128), ("acrobot", 32): (16, 128), ("acrobot", 64): (16, None)}
+
+
+@pytest.mark.parametrize("body,hidden", sorted(_FORM_BOUNDS))
+def test_every_starting_form_gives_the_same_scores(dev, body, hidden):
+    """Populations just past each bound of the launch rule (ragged last waves) against the same
+    members run in slices small enough for the 16-lane form, which the tests above pin to the
+    oracle: every member's score equal, whatever forms its wave went through."""
+    from hipenvs import acrobot_rollout, cartpole_rollout
+
+    mod = cartpole_rollout if body == "cartpole" else acrobot_rollout
+    reset = oc.reset if body == "cartpole" else oa.reset
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    b16, b4 = _FORM_BOUNDS[body, hidden]
+    p = (b4 or 2 * b16) * cus + 37
+    horizon = 150 if body == "cartpole" else 90
+    theta = torch.from_numpy(_mixed_population(body, p, hidden, 7 + hidden)).to(dev)
+    state = torch.from_numpy(reset(p, seed=11)).to(dev)
+    want = torch.cat([mod.rollout_steps(state[:, a:a + 4001].contiguous(), theta[a:a + 4001], hidden, horizon)
+                      for a in range(0, p, 4001)])
+    for n in (p, b16 * cus + 1, b16 * cus):
+        got = mod.rollout_steps(state[:, :n].contiguous(), theta[:n], hidden, horizon)
+        assert torch.equal(got, want[:n]), n
+    assert len(want.unique()) > 3  # members ended at many different steps
+    one = mod.rollout_steps(state[:, :1].contiguous(), theta[:1], hidden, horizon)
+    assert torch.equal(one, want[:1])
+    for h in (0, 1):  # nothing to step; the horizon reached in the first form
+        got = mod.rollout_steps(state, theta, hidden, h)
+        assert torch.equal(got, torch.clamp(want, max=h))
+
+
+def test_shared_policy_takes_every_starting_form(dev):
+    """The greedy evaluation (member stride 0) past the lane-group bounds equals its slices."""
+    from hipenvs import acrobot_rollout, cartpole_rollout
+
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    n = 130 * cus + 3
+    for mod, reset, d in ((cartpole_rollout, oc.reset, 7 * 8 + 2), (acrobot_rollout, oa.reset, 10 * 8 + 3)):
+        theta = torch.from_numpy(population(2, d, 3, scale=0.4)[0]).to(dev)
+        state = torch.from_numpy(reset(n, seed=2)).to(dev)
+        got = mod.evaluate(state, theta, 8, 80)
+        want = torch.cat([mod.evaluate(state[:, a:a + 4000].contiguous(), theta, 8, 80) for a in range(0, n, 4000)])
+        assert torch.equal(got, want)
 
 
 def test_config2_cartpole_population(dev):
