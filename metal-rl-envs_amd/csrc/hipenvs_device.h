@@ -251,7 +251,7 @@ __device__ __forceinline__ void det_sincos_all(const float* x, float* sin_out, f
 // with an initialised old value, which costs a v_mov per broadcast).
 template <int L>
 __device__ __forceinline__ float group_bcast(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + L, 0xF, 0xF, false));
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + L, 0xF, 0xF, true));
 }
 
 // Lane L (< 8) of each 8-lane half of every 16-lane row, on every lane of that half: how an
@@ -278,7 +278,7 @@ __device__ __forceinline__ float lane_bcast(float v) {
     return half_bcast<L>(v);
   } else {
     static_assert(L >= 0 && L < 4, "a lane of the quad");
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), L * 0x55, 0xF, 0xF, false));
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), L * 0x55, 0xF, 0xF, true));
   }
 }
 
@@ -435,6 +435,7 @@ __device__ __forceinline__ float sqrt_pivot(float s, double* recip_out) {
 }
 
 struct DivRecip {
+  static constexpr bool kRecip = true;  // divides by multiplying with r; d is not read
   // Per lane, the least (bits << 1) - 2 over the quotients, in uint32 arithmetic: the shift
   // drops the sign, and the subtraction sends zero to the top, so a nonzero subnormal
   // (0 < |bits| <= 0x7FFFFF) maps to at most 0xFFFFFC and every other value above it. One
@@ -450,6 +451,7 @@ struct DivRecip {
 };
 
 struct DivIEEE {
+  static constexpr bool kRecip = false;
   __device__ __forceinline__ float operator()(float a, float d, double /*r*/) const { return a / d; }
 };
 

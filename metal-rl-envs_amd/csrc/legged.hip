@@ -1,17 +1,8 @@
-// The C-legged body with hard ground contacts on MI355X: the env step and the
-// fused legged ES rollout, one thread per environment, everything in VGPRs.
-//
-// Physics: legged_np.py:57-97 in float32, operation by operation. Per substep:
-// foot Jacobians (C sincos), the (3+C)^2 mass matrix, a dense Cholesky reused
-// for the free velocity and the 2C columns M^-1 J^T, the C^2 Delassus blocks,
-// `iters` sweeps of block projected Gauss-Seidel with the exact single-contact
-// solve (hopper_np.py:80-109), semi-implicit Euler. Terms the reference
-// multiplies by an exact zero or one are elided where that leaves every value
-// unchanged (x * 1 = x, x + (+-0) = x); the order of every remaining operation
-// is numpy's.
+// The fused rollouts of the C-legged body: ES populations (the caller's weights or
+// regenerated from a seed) and the greedy evaluation.
 //
 // The rollout runs each member's (5+2C)-H-3C tanh policy (one three-way head
-// per leg) and the physics for the whole horizon (legged_rollout_metal.py:19-59).
+// per leg) and the physics (legged_body.h) for the whole horizon (legged_rollout_metal.py:19-59).
 // The member's weights are streamed from memory every step (D = 1,676 floats at
 // C = 4, H = 64 do not fit in registers), either from es.unflatten's rows
 // (P, D) or from a column layout (D, P) in which a wave's 64 members read 256
@@ -20,603 +11,10 @@
 #include <type_traits>
 
 #include "es_noise.h"
+#include "legged_body.h"
 
 namespace hipenvs {
 namespace lg {
-
-constexpr float M_F = 0x1.99999ap-3f;              // float32(0.2)
-constexpr float I_T = 0x1.99999ap-4f;              // float32(0.1)
-constexpr float GRAVITY = 0x1.39999ap+3f;          // float32(9.8)
-constexpr float NEG_M_F = -0x1.99999ap-3f;         // float32(-0.2)
-constexpr float H = 0x1.47ae14p-7f;                // float32(0.01)
-constexpr float MU = 0x1.666666p-1f;               // float32(0.7)
-constexpr float BAUMGARTE_OVER_H = 0x1.4p+4f;      // float32(0.2 / 0.01)
-constexpr float FALL_HEIGHT = 0x1.333334p-1f;      // float32(0.6)
-constexpr float FALL_ANGLE = 0x1p+0f;              // float32(1.0)
-constexpr float RESET_BOUND = 0x1.99999ap-5f;      // float32(0.05)
-constexpr float TORQUE = 0x1p+1f;                  // float32(2.0)
-constexpr int SUBSTEPS = 4;
-
-// np.maximum(x, 0.0): NaN propagates.
-__device__ __forceinline__ float max0(float x) { return (x < 0.0f) ? 0.0f : x; }
-
-// Exact impulse of one contact given its Delassus block and relative velocity
-// (hopper_np.py:80-109), float32 throughout.
-// The per-substep constants of one contact's diagonal Delassus block: the 2x2 determinant
-// and the two cone-edge denominators with their float64 reciprocals, formed once per
-// substep instead of once per sweep (the values are the same float32 numbers either way).
-struct ContactBlock {
-  float Att, Atn, Ann, det, den_p, den_m;
-  double rdet, rden_p, rden_m;
-};
-
-__device__ __forceinline__ ContactBlock contact_block(float Att, float Atn, float Ann) {
-  ContactBlock b;
-  b.Att = Att;
-  b.Atn = Atn;
-  b.Ann = Ann;
-  b.det = Att * Ann - Atn * Atn;
-  b.den_p = Ann + MU * Atn;
-  b.den_m = Ann - MU * Atn;
-  b.rdet = recip(b.det);
-  b.rden_p = recip(b.den_p);
-  b.rden_m = recip(b.den_m);
-  return b;
-}
-
-template <class Div>
-__device__ __forceinline__ void contact_impulse(const ContactBlock& b, float wt, float wn, float depth,
-                                                float& lt_out, float& ln_out, Div& div) {
-  const float Att = b.Att, Atn = b.Atn, Ann = b.Ann;
-  const bool touching = depth >= 0.0f;
-  const float target = BAUMGARTE_OVER_H * max0(depth);
-  const float tw = target - wn;
-  const float ln_stick = div(Att * tw + Atn * wt, b.det, b.rdet);
-  const float lt_stick = div((-Ann) * wt - Atn * tw, b.det, b.rdet);
-  const bool sticks = fabsf(lt_stick) <= MU * ln_stick;
-  // both cone quotients are formed whatever the signs of their denominators and selected
-  // after (no branch); a subnormal mark from an unused one only costs an exact redo
-  const float q_p = div(tw, b.den_p, b.rden_p);
-  const float q_m = div(tw, b.den_m, b.rden_m);
-  const float ln_p = (b.den_p > 0.0f) ? max0(q_p) : 0.0f;
-  const float ln_m = (b.den_m > 0.0f) ? max0(q_m) : 0.0f;
-  const float slip_p = wt + (Att * MU + Atn) * ln_p;
-  const float s = (slip_p <= 0.0f) ? 1.0f : -1.0f;
-  const float ln_slide = (slip_p <= 0.0f) ? ln_p : ln_m;
-  const float lt_slide = (MU * s) * ln_slide;
-  const float ln = sticks ? ln_stick : ln_slide;
-  const float lt = sticks ? lt_stick : lt_slide;
-  const bool active = touching && (ln > 0.0f) && (wn < target);
-  lt_out = active ? lt : 0.0f;
-  ln_out = active ? ln : 0.0f;
-}
-
-// Solve L L^T x = b in place (pendulum_np.py:95-107): forward then backward substitution.
-// rL[i] = recip(L[i][i]): the 2N divisions of a solve share the N diagonal reciprocals.
-template <int N, class Div>
-__device__ __forceinline__ void chol_solve(const float (&L)[N][N], const double (&rL)[N], float (&b)[N], Div& div) {
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    float s = b[i];
-#pragma unroll
-    for (int p = 0; p < i; ++p) s = s - L[i][p] * b[p];
-    b[i] = div(s, L[i][i], rL[i]);
-  }
-#pragma unroll
-  for (int i = N - 1; i >= 0; --i) {
-    float s = b[i];
-#pragma unroll
-    for (int p = i + 1; p < N; ++p) s = s - L[p][i] * b[p];
-    b[i] = div(s, L[i][i], rL[i]);
-  }
-}
-
-// sa[k], ca[k] = lane k's sn, cs, for k < K, on every lane of the G-lane group.
-template <int G, int K>
-__device__ __forceinline__ void row_trig(float sn, float cs, float* sa, float* ca) {
-  if constexpr (K > 0) {
-    row_trig<G, K - 1>(sn, cs, sa, ca);
-    sa[K - 1] = lane_bcast<G, K - 1>(sn);
-    ca[K - 1] = lane_bcast<G, K - 1>(cs);
-  }
-}
-
-// out[i] = lane i's x, for i < K, on every lane of the G-lane group.
-template <int G, int K>
-__device__ __forceinline__ void row_gather(float x, float* out) {
-  if constexpr (K > 0) {
-    row_gather<G, K - 1>(x, out);
-    out[K - 1] = lane_bcast<G, K - 1>(x);
-  }
-}
-
-// One semi-implicit Euler substep with block PGS contacts, in place (legged_np.py:57-97).
-// kGroup = 0: one lane computes the whole substep. kGroup = G (8 or 16): the G lanes
-// g = 0..G-1 of a member's group (a 16-lane DPP row or half of one) all hold the member's
-// state and compute everything identically, except that lane g < C evaluates foot g's sin
-// and cos, shared by DPP broadcast, the Gauss-Seidel sweeps and the velocity update split
-// their independent work over the lanes (below), and lane g solves right-hand sides g,
-// g + G, ... of the 2C + 1 triangular solves
-// (the forces, then the tangent, then the normal Jacobian rows), exchanged through the
-// group's LDS rows xs ((2C + 1) x 8 floats). Every value is computed by the same expression
-// as in the one-lane form, so the results are the same bits. Callers keep the group's
-// lanes in one single-wave workgroup, so the barriers order its LDS traffic.
-// kHopperSum (C = 1 only) adds the impulse terms as the reference's hopper does,
-// (v_free + M^-1 J_t^T lt) + M^-1 J_n^T ln (hopper_np.py:76), instead of the legged body's
-// v_free + (M^-1 J_t^T lt + M^-1 J_n^T ln) (legged_np.py:95); otherwise the hopper is this
-// body at C = 1 with one sweep.
-// kStage (one-lane form only) parks the M^-1 J^T columns in LDS during the Gauss-Seidel
-// sweeps, at xs[e * 64] for element e (xs points at the lane's own column of a 64-lane
-// block), which frees 2C(3 + C) registers there; they are read back for the velocity update.
-template <int C, class Div, int kGroup = 0, bool kHopperSum = false, bool kStage = false>
-__device__ __forceinline__ void substep(float (&q)[3 + C], float (&v)[3 + C], const float (&tq)[C], int iters,
-                                        float assist, float assist_damping, Div& div, float* xs = nullptr,
-                                        int g = 0, float* xd = nullptr) {
-  constexpr int N = 3 + C;
-  float ca[C], sa[C], dx[C], dy[C], depth[C], r2[C];
-  if constexpr (kGroup >= 4 && kGroup >= C) {
-    // lane g < C evaluates foot g's sin and cos, shared by DPP broadcast within the group
-    static_assert(C <= kGroup, "one lane per foot");
-    float a = q[2] + q[3];
-#pragma unroll
-    for (int k = 1; k < C; ++k) a = (g == k) ? q[2] + q[3 + k] : a;
-    float sn, cs;
-    det_sincos(a, &sn, &cs);
-    row_trig<kGroup, C>(sn, cs, sa, ca);
-  } else {
-#pragma unroll
-    for (int k = 0; k < C; ++k) det_sincos(q[2] + q[3 + k], &sa[k], &ca[k]);
-  }
-#pragma unroll
-  for (int k = 0; k < C; ++k) {
-    const float ad = v[2] + v[3 + k];
-    dx[k] = ((-sa[k]) * ad) * ad;
-    dy[k] = (ca[k] * ad) * ad;
-    depth[k] = -(q[1] - ca[k]);
-    r2[k] = ca[k] * ca[k] + sa[k] * sa[k];
-  }
-  // sums over the feet in the reference's order
-  float s_ca = ca[0], s_sa = sa[0], s_r2 = r2[0], s_dx = dx[0], s_dy = dy[0], s_f2 = ca[0] * dx[0] + sa[0] * dy[0];
-#pragma unroll
-  for (int k = 1; k < C; ++k) {
-    s_ca = s_ca + ca[k];
-    s_sa = s_sa + sa[k];
-    s_r2 = s_r2 + r2[k];
-    s_dx = s_dx + dx[k];
-    s_dy = s_dy + dy[k];
-    s_f2 = s_f2 + (ca[k] * dx[k] + sa[k] * dy[k]);
-  }
-  // mass matrix, lower triangle (M_T = 1: base 1 + M_F * C on x and y)
-  float L[N][N];
-  const float mxy = 1.0f + M_F * (float)C;
-  L[0][0] = mxy;
-  L[1][0] = M_F * 0.0f;
-  L[1][1] = mxy;
-  L[2][0] = M_F * s_ca;
-  L[2][1] = M_F * s_sa;
-  L[2][2] = I_T + M_F * s_r2;
-#pragma unroll
-  for (int j = 0; j < C; ++j) {
-    L[3 + j][0] = M_F * ca[j];
-    L[3 + j][1] = M_F * sa[j];
-    L[3 + j][2] = M_F * r2[j];
-#pragma unroll
-    for (int i = 0; i < j; ++i) L[3 + j][3 + i] = M_F * 0.0f;
-    L[3 + j][3 + j] = M_F * r2[j];
-  }
-  // generalised forces: bias, gravity, leg torques, torso assist
-  float f[N];
-  f[0] = NEG_M_F * s_dx;
-  f[1] = NEG_M_F * s_dy - GRAVITY * (M_F * (float)C + 1.0f);
-  f[2] = NEG_M_F * s_f2 - GRAVITY * (M_F * s_sa);
-#pragma unroll
-  for (int j = 0; j < C; ++j) {
-    f[3 + j] = NEG_M_F * (ca[j] * dx[j] + sa[j] * dy[j]) - GRAVITY * (M_F * sa[j]);
-    f[3 + j] = f[3 + j] + tq[j];
-  }
-  f[2] = (f[2] - assist * q[2]) - assist_damping * v[2];
-  // Cholesky in place (pendulum_np.py:88-94), keeping each pivot's float64 reciprocal
-  double rL[N];
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-#pragma unroll
-    for (int j = 0; j <= i; ++j) {
-      float s = L[i][j];
-#pragma unroll
-      for (int p = 0; p < j; ++p) s = s - L[i][p] * L[j][p];
-      if (i == j) {
-        L[i][i] = sqrt_pivot(s, &rL[i]);
-      } else {
-        L[i][j] = div(s, L[j][j], rL[j]);
-      }
-    }
-  }
-  // M^-1 f and the M^-1 J^T columns
-  float MiJt[C][N], MiJn[C][N];
-  if constexpr (kGroup == 0) {
-    chol_solve<N>(L, rL, f, div);
-#pragma unroll
-    for (int k = 0; k < C; ++k) {
-#pragma unroll
-      for (int i = 0; i < N; ++i) {
-        MiJt[k][i] = (i == 0) ? 1.0f : (i == 2 || i == 3 + k) ? ca[k] : 0.0f;
-        MiJn[k][i] = (i == 1) ? 1.0f : (i == 2 || i == 3 + k) ? sa[k] : 0.0f;
-      }
-      chol_solve<N>(L, rL, MiJt[k], div);
-      chol_solve<N>(L, rL, MiJn[k], div);
-    }
-  } else {
-    constexpr int kRow = 8;  // LDS floats per right-hand side
-    constexpr int kRhs = 2 * C + 1, kRounds = (kRhs + kGroup - 1) / kGroup;
-    float b[kRounds][N];
-#pragma unroll
-    for (int r = 0; r < kRounds; ++r) {
-      // lane g solves right-hand sides g, g + kGroup, ...; past 2C it solves the forces again, unused
-      const int rhs = g + r * kGroup < kRhs ? g + r * kGroup : 0;
-      const bool normal = rhs > C;
-      const int k = normal ? rhs - 1 - C : rhs - 1;
-      float ck = ca[0], sk = sa[0];
-#pragma unroll
-      for (int kk = 1; kk < C; ++kk) {
-        ck = (k == kk) ? ca[kk] : ck;
-        sk = (k == kk) ? sa[kk] : sk;
-      }
-#pragma unroll
-      for (int i = 0; i < N; ++i) {
-        const bool on = (i == 2 || i == 3 + k);
-        const float jt = (i == 0) ? 1.0f : on ? ck : 0.0f;
-        const float jn = (i == 1) ? 1.0f : on ? sk : 0.0f;
-        b[r][i] = (rhs == 0) ? f[i] : normal ? jn : jt;
-      }
-      chol_solve<N>(L, rL, b[r], div);
-    }
-    __syncthreads();  // the rows' previous readers are done
-#pragma unroll
-    for (int r = 0; r < kRounds; ++r) {
-      if (g + r * kGroup < kRhs) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) xs[(g + r * kGroup) * kRow + i] = b[r][i];
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < N; ++i) f[i] = xs[i];
-    // the M^-1 J^T columns stay in xs until the velocity update reads them
-  }
-  float vf[N];
-#pragma unroll
-  for (int i = 0; i < N; ++i) vf[i] = v[i] + H * f[i];
-  // Delassus blocks A[k][l] = (Jt_k.MiJt_l, Jt_k.MiJn_l, Jn_k.MiJt_l, Jn_k.MiJn_l) and free velocities
-  float Att[C][C], Atn[C][C], Ant[C][C], Ann[C][C], w0t[C], w0n[C];
-  if constexpr (kGroup > 0) {
-    // lane g < C^2 forms block (g / C, g % C) from the solved rows in xs, and a lane of a
-    // diagonal block also forms its contact's ContactBlock; the group reads the C^2 blocks
-    // (4 floats each) and the C contact blocks (12 floats each) back from xd
-    constexpr int kRow = 8;
-    constexpr int kBlocks = C * C, kRounds = (kBlocks + kGroup - 1) / kGroup;
-#pragma unroll
-    for (int r = 0; r < kRounds; ++r) {
-      const int gr = g + r * kGroup;
-      const int gb = gr < kBlocks ? gr : 0;  // lanes past C^2 form block 0 again, unused
-      const int kb = gb / C, lb = gb % C;
-      float ck = ca[0], sk = sa[0];
-#pragma unroll
-      for (int kk = 1; kk < C; ++kk) {
-        ck = (kb == kk) ? ca[kk] : ck;
-        sk = (kb == kk) ? sa[kk] : sk;
-      }
-      const float* rt = xs + (1 + lb) * kRow;
-      const float* rn = xs + (1 + C + lb) * kRow;
-      const float t2 = rt[2], t3 = rt[3 + kb], n2 = rn[2], n3 = rn[3 + kb];
-      const float4 blk4 = make_float4((rt[0] + ck * t2) + ck * t3, (rn[0] + ck * n2) + ck * n3,
-                                      (rt[1] + sk * t2) + sk * t3, (rn[1] + sk * n2) + sk * n3);
-      if (gr < kBlocks) *reinterpret_cast<float4*>(xd + 4 * gr) = blk4;
-      const ContactBlock own = contact_block(blk4.x, blk4.y, blk4.w);
-      if (gr < kBlocks && kb == lb) {
-        float* xc = xd + 4 * C * C + 12 * kb;
-        *reinterpret_cast<float4*>(xc) = make_float4(own.det, own.den_p, own.den_m, 0.0f);
-        *reinterpret_cast<double2*>(xc + 4) = make_double2(own.rdet, own.rden_p);
-        *reinterpret_cast<double*>(xc + 8) = own.rden_m;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < C; ++k) {
-#pragma unroll
-      for (int l = 0; l < C; ++l) {
-        const float4 e = *reinterpret_cast<const float4*>(xd + 4 * (k * C + l));
-        Att[k][l] = e.x;
-        Atn[k][l] = e.y;
-        Ant[k][l] = e.z;
-        Ann[k][l] = e.w;
-      }
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < C; ++k) {
-#pragma unroll
-      for (int l = 0; l < C; ++l) {
-        Att[k][l] = (MiJt[l][0] + ca[k] * MiJt[l][2]) + ca[k] * MiJt[l][3 + k];
-        Atn[k][l] = (MiJn[l][0] + ca[k] * MiJn[l][2]) + ca[k] * MiJn[l][3 + k];
-        Ant[k][l] = (MiJt[l][1] + sa[k] * MiJt[l][2]) + sa[k] * MiJt[l][3 + k];
-        Ann[k][l] = (MiJn[l][1] + sa[k] * MiJn[l][2]) + sa[k] * MiJn[l][3 + k];
-      }
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < C; ++k) {
-    w0t[k] = (vf[0] + ca[k] * vf[2]) + ca[k] * vf[3 + k];
-    w0n[k] = (vf[1] + sa[k] * vf[2]) + sa[k] * vf[3 + k];
-  }
-  if constexpr (kStage) {
-    static_assert(kGroup == 0, "staging is for the one-lane form");
-#pragma unroll
-    for (int k = 0; k < C; ++k) {
-#pragma unroll
-      for (int i = 0; i < N; ++i) {
-        xs[(k * N + i) * 64] = MiJt[k][i];
-        xs[((C + k) * N + i) * 64] = MiJn[k][i];
-      }
-    }
-    asm volatile("" ::: "memory");  // the columns live in LDS until the velocity update
-  }
-  // block projected Gauss-Seidel, fixed contact order (legged_np.py:88-93)
-  float lt[C], ln[C];
-  ContactBlock blk[C];
-#pragma unroll
-  for (int k = 0; k < C; ++k) {
-    lt[k] = 0.0f;
-    ln[k] = 0.0f;
-    if constexpr (kGroup > 0) {
-      const float* xc = xd + 4 * C * C + 12 * k;
-      const float4 f4 = *reinterpret_cast<const float4*>(xc);
-      const double2 d2 = *reinterpret_cast<const double2*>(xc + 4);
-      blk[k] = ContactBlock{Att[k][k], Atn[k][k], Ann[k][k], f4.x, f4.y, f4.z,
-                            d2.x, d2.y, *reinterpret_cast<const double*>(xc + 8)};
-    } else {
-      blk[k] = contact_block(Att[k][k], Atn[k][k], Ann[k][k]);
-    }
-  }
-  if constexpr (kGroup >= 4) {
-    // The member's lanes split each contact's independent work and share the results by
-    // DPP broadcast: lane 1 forms the normal coupling sum and every other lane the tangential
-    // one (each with its own coefficient rows), and lanes 0-3 form the four quotients of the
-    // contact solve, ln_stick, lt_stick, (target - wn) / den_p and (target - wn) / den_m
-    // (lanes 4 and up repeat lane 0's). Every broadcast value is the expression the one-lane
-    // sweep evaluates, so the impulses are the same bits.
-    // Each lane reads its own coefficients from the group's LDS blocks at a lane-dependent
-    // offset (block (k, l) holds Att, Atn, Ant, Ann; contact k's block holds det, den_p,
-    // den_m and then their float64 reciprocals), and negates by flipping the sign bit: no
-    // per-lane selects, which the compiler had turned into exec-mask branches.
-    const bool nrow = (g == 1);
-    const int sel = (g == 2) ? 1 : (g == 3) ? 2 : 0;       // det, den_p, den_m
-    const uint32_t neg = nrow ? 0x80000000u : 0u;
-    const int oA = nrow ? 2 : 0, oB = nrow ? 3 : 1, oQ = nrow ? 1 : 0;  // Ant|Att, Ann|Atn, Atn|Att
-    // Lanes 2 and 3 clamp their cone-edge quotients before the broadcast, as the contact solve
-    // does after it: (den > 0) ? max0(q) : 0, that is 0 where den > 0 fails or q < 0, else q
-    // (-0 and NaN pass, as in max0). Lanes 0 and 1 compare against -inf, which nothing is
-    // below, and pass their stick quotients on unchanged. One clamp on two lanes replaces two
-    // on every lane. No mask on the chain from the quotients to the impulses is combined on
-    // the scalar unit, which would wait for the vector compare to complete: the gate's mask
-    // is formed before the quotients, and the clamp and the gate are each one compare.
-    const bool edge = (g == 2 || g == 3);
-    const float qlo = edge ? 0.0f : -__builtin_inff();
-    float cA[C][C], cB[C][C], w0x[C], qP[C], qQ[C], qd[C], slipc[C];
-    bool qzero[C];
-    double qr[C];
-#pragma unroll
-    for (int k = 0; k < C; ++k) {
-#pragma unroll
-      for (int l = 0; l < C; ++l) {
-        cA[k][l] = xd[4 * (k * C + l) + oA];
-        cB[k][l] = xd[4 * (k * C + l) + oB];
-      }
-      w0x[k] = nrow ? w0n[k] : w0t[k];
-      // numerators qP * wt + qQ * tw: lane 0 Atn wt + Att tw, which is the reference's
-      // Att tw + Atn wt (a rounded sum commutes); lane 1 (-Ann) wt + (-Atn) tw, which is
-      // the reference's (-Ann) wt - Atn tw exactly (a - b = a + (-b))
-      const float* xb = xd + 4 * (k * C + k);
-      qP[k] = __uint_as_float(__float_as_uint(xb[oB]) ^ neg);
-      qQ[k] = __uint_as_float(__float_as_uint(xb[oQ]) ^ neg);
-      const float* xc = xd + 4 * C * C + 12 * k;
-      qd[k] = xc[sel];
-      qr[k] = *reinterpret_cast<const double*>(xc + 4 + 2 * sel);
-      qzero[k] = edge && !(qd[k] > 0.0f);  // lane 2 holds den_p, lane 3 den_m
-      // such a lane divides -1 by 1 instead, whose quotient the clamp sets to 0: the clamp
-      // then needs no mask of its own (a mask combined on the scalar unit between the
-      // quotient and its broadcast waits for the vector compare)
-      qd[k] = qzero[k] ? 1.0f : qd[k];
-      qr[k] = qzero[k] ? 1.0 : qr[k];
-      slipc[k] = blk[k].Att * MU + blk[k].Atn;
-    }
-    // -1 in a register the compiler cannot see through: an impulse whose contact is not
-    // pushing (open below) is gated as max(-1, ...) would be, by one compare of a select
-    // rather than two compares combined on the scalar unit
-    float neg_one = -1.0f;
-    asm volatile("" : "+v"(neg_one));
-    for (int it = 0; it < iters; ++it) {
-#pragma unroll
-      for (int k = 0; k < C; ++k) {
-        float wt, wn;
-        if constexpr (C == 1) {
-          wt = w0t[k];
-          wn = w0n[k];
-        } else {
-          float sx = 0.0f;
-          bool first = true;
-#pragma unroll
-          for (int l = 0; l < C; ++l) {
-            if (l == k) continue;
-            const float tx = cA[k][l] * lt[l] + cB[k][l] * ln[l];
-            sx = first ? tx : sx + tx;
-            first = false;
-          }
-          const float wx = w0x[k] + sx;
-          wt = lane_bcast<kGroup, 0>(wx);
-          wn = lane_bcast<kGroup, 1>(wx);
-        }
-        const bool touching = depth[k] >= 0.0f;
-        const float target = BAUMGARTE_OVER_H * max0(depth[k]);
-        const float tw = target - wn;
-        const bool open = touching && (wn < target);  // known before the quotients
-        const float num = qzero[k] ? -1.0f : edge ? tw : qP[k] * wt + qQ[k] * tw;
-        const float quo = div(num, qd[k], qr[k]);
-        const float qc = (quo < qlo) ? 0.0f : quo;
-        const float ln_stick = lane_bcast<kGroup, 0>(qc);
-        const float lt_stick = lane_bcast<kGroup, 1>(qc);
-        const float ln_p = lane_bcast<kGroup, 2>(qc);
-        const float ln_m = lane_bcast<kGroup, 3>(qc);
-        const bool sticks = fabsf(lt_stick) <= MU * ln_stick;
-        const float slip_p = wt + slipc[k] * ln_p;
-        const float sgn = (slip_p <= 0.0f) ? 1.0f : -1.0f;
-        const float ln_slide = (slip_p <= 0.0f) ? ln_p : ln_m;
-        const float lt_slide = (MU * sgn) * ln_slide;
-        const float lnv = sticks ? ln_stick : ln_slide;
-        const float ltv = sticks ? lt_stick : lt_slide;
-        const bool active = (open ? lnv : neg_one) > 0.0f;  // open && lnv > 0
-        lt[k] = active ? ltv : 0.0f;
-        ln[k] = active ? lnv : 0.0f;
-      }
-    }
-  } else {
-    for (int it = 0; it < iters; ++it) {
-#pragma unroll
-      for (int k = 0; k < C; ++k) {
-        float st = 0.0f, sn = 0.0f;
-        bool first = true;
-#pragma unroll
-        for (int l = 0; l < C; ++l) {
-          if (l == k) continue;
-          const float tt = Att[k][l] * lt[l] + Atn[k][l] * ln[l];
-          const float nn = Ant[k][l] * lt[l] + Ann[k][l] * ln[l];
-          st = first ? tt : st + tt;
-          sn = first ? nn : sn + nn;
-          first = false;
-        }
-        const float wt = (C == 1) ? w0t[k] : w0t[k] + st;
-        const float wn = (C == 1) ? w0n[k] : w0n[k] + sn;
-        contact_impulse(blk[k], wt, wn, depth[k], lt[k], ln[k], div);
-      }
-    }
-  }
-  // v = v_free + sum_k M^-1 J_k^T lambda_k; q += h v
-  if constexpr (kStage) {
-    asm volatile("" ::: "memory");
-#pragma unroll
-    for (int k = 0; k < C; ++k) {
-#pragma unroll
-      for (int i = 0; i < N; ++i) {
-        MiJt[k][i] = xs[(k * N + i) * 64];
-        MiJn[k][i] = xs[((C + k) * N + i) * 64];
-      }
-    }
-  } else if constexpr (kGroup >= 3 + C && !kHopperSum) {
-    // lane i < N forms velocity i (its sum over the contacts in the same order as below,
-    // from its own column of the solved rows) and the DPP broadcast gives it to the group
-    static_assert(3 + C <= kGroup, "one lane per velocity");
-    constexpr int kRow = 8;
-    asm volatile("" ::: "memory");  // read here, not held in registers through the sweeps
-    const int i = g < N ? g : 0;  // lanes past N form velocity 0 again, unused
-    float vfi = vf[0];
-#pragma unroll
-    for (int r = 1; r < N; ++r) vfi = (i == r) ? vf[r] : vfi;
-    float si = xs[(1 + 0) * kRow + i] * lt[0] + xs[(1 + C + 0) * kRow + i] * ln[0];
-#pragma unroll
-    for (int k = 1; k < C; ++k) si = si + (xs[(1 + k) * kRow + i] * lt[k] + xs[(1 + C + k) * kRow + i] * ln[k]);
-    float vn[N];
-    row_gather<kGroup, N>(vfi + si, vn);
-#pragma unroll
-    for (int r = 0; r < N; ++r) {
-      v[r] = vn[r];
-      q[r] = q[r] + H * vn[r];
-    }
-    return;
-  } else if constexpr (kGroup > 0) {
-    constexpr int kRow = 8;
-    asm volatile("" ::: "memory");  // read here, not held in registers through the sweeps
-#pragma unroll
-    for (int k = 0; k < C; ++k) {
-#pragma unroll
-      for (int i = 0; i < N; ++i) {
-        MiJt[k][i] = xs[(1 + k) * kRow + i];
-        MiJn[k][i] = xs[(1 + C + k) * kRow + i];
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    float vn;
-    if constexpr (kHopperSum) {
-      static_assert(C == 1, "the hopper has one contact");
-      vn = (vf[i] + MiJt[0][i] * lt[0]) + MiJn[0][i] * ln[0];
-    } else {
-      float s = MiJt[0][i] * lt[0] + MiJn[0][i] * ln[0];
-#pragma unroll
-      for (int k = 1; k < C; ++k) s = s + (MiJt[k][i] * lt[k] + MiJn[k][i] * ln[k]);
-      vn = vf[i] + s;
-    }
-    v[i] = vn;
-    q[i] = q[i] + H * vn;
-  }
-}
-
-// One substep dividing through the shared float64 reciprocals; a lane on which a quotient
-// came out subnormal (never met in practice) redoes the substep from its saved state with
-// IEEE division, so the result is always the IEEE one.
-template <int C, bool kHopperSum = false, bool kStage = false>
-__device__ __forceinline__ void substep_exact(float (&q)[3 + C], float (&v)[3 + C], const float (&tq)[C], int iters,
-                                              float assist, float assist_damping, float* stage = nullptr) {
-  constexpr int N = 3 + C;
-  float q0[N], v0[N];
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    q0[i] = q[i];
-    v0[i] = v[i];
-  }
-  DivRecip fast;
-  substep<C, DivRecip, 0, kHopperSum, kStage>(q, v, tq, iters, assist, assist_damping, fast, stage);
-  if (fast.saw_subnormal()) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      q[i] = q0[i];
-      v[i] = v0[i];
-    }
-    DivIEEE ieee;
-    substep<C, DivIEEE, 0, kHopperSum, kStage>(q, v, tq, iters, assist, assist_damping, ieee, stage);
-  }
-}
-
-// The group form of substep_exact: the fast divisions, and when any live lane of the wave saw
-// a subnormal quotient the whole wave redoes the substep with IEEE division (identical bits
-// wherever nothing was marked), which keeps the group's barriers in uniform control flow.
-template <int C, int G>
-__device__ __forceinline__ void substep_exact_group(float (&q)[3 + C], float (&v)[3 + C], const float (&tq)[C],
-                                                    int iters, float assist, float assist_damping, float* xs, int g,
-                                                    bool live, float* xd) {
-  constexpr int N = 3 + C;
-  float q0[N], v0[N];
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    q0[i] = q[i];
-    v0[i] = v[i];
-  }
-  DivRecip fast;
-  substep<C, DivRecip, G>(q, v, tq, iters, assist, assist_damping, fast, xs, g, xd);
-  if (__any(live && fast.saw_subnormal())) {  // lanes of finished members step on, unused
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      q[i] = q0[i];
-      v[i] = v0[i];
-    }
-    DivIEEE ieee;
-    substep<C, DivIEEE, G>(q, v, tq, iters, assist, assist_damping, ieee, xs, g, xd);
-  }
-}
-
-template <int C>
-__device__ __forceinline__ bool fallen(const float (&q)[3 + C]) {
-  return (q[1] < FALL_HEIGHT) || (fabsf(q[2]) > FALL_ANGLE);
-}
 
 // Minimum resident waves per SIMD the rollout kernels are compiled for (bounds their VGPRs).
 #ifndef LEGGED_ROLLOUT_MIN_WAVES
@@ -913,83 +311,6 @@ __device__ __forceinline__ void policy_group(const float* __restrict__ w, const 
   }
 }
 
-// kHopper (C = 1): the reference's hopper step (hopper_metal.py:84-125): torque
-// (a - 1) * TORQUE for any action value, its impulse sum order, and the standing pose
-// (0, L, 0, 0) with zero velocities built in (stand is not read).
-template <int C, bool kHopper = false>
-__global__ __launch_bounds__(kBlock) void step_kernel(const float* __restrict__ state,
-                                                      const int32_t* __restrict__ action, uint32_t seed,
-                                                      const float* __restrict__ stand, int iters, float assist,
-                                                      float assist_damping, float* __restrict__ next,
-                                                      float* __restrict__ reward, uint8_t* __restrict__ done,
-                                                      int64_t n) {
-  constexpr int N = 3 + C;
-  const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (e >= n) return;
-  float q[N], v[N], tq[C];
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    q[i] = state[i * n + e];
-    v[i] = state[(N + i) * n + e];
-  }
-  // leg k gets ((a / 3^k) % 3 - 1) * TORQUE (legged_np.py:51-54)
-  int32_t a = stream_load(action + e);
-  if constexpr (kHopper) {
-    tq[0] = (float)(a - 1) * TORQUE;
-  } else {
-#pragma unroll
-    for (int k = 0; k < C; ++k) {
-      tq[k] = (float)(a % 3 - 1) * TORQUE;
-      a /= 3;
-    }
-  }
-#pragma unroll 1
-  for (int s = 0; s < SUBSTEPS; ++s) substep_exact<C, kHopper>(q, v, tq, iters, assist, assist_damping);
-  const bool d = fallen<C>(q);
-  stream_store(d ? 0.0f : v[0] + 1.0f, reward + e);
-  stream_store((uint8_t)(d ? 1 : 0), done + e);
-  if (d) {  // fresh draws only on fallen lanes; the reference selects (legged_metal.py:148-152)
-    const uint32_t h = env_hash(seed, (uint32_t)e);
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      const float pose = kHopper ? (i == 1 ? 1.0f : 0.0f) : stand[i];  // hopper: y = L = 1
-      q[i] = pose + uniform_pm(pcg_hash(h + (uint32_t)i * kRowStride), RESET_BOUND);
-    }
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      const float pose = kHopper ? 0.0f : stand[N + i];
-      v[i] = pose + uniform_pm(pcg_hash(h + (uint32_t)(N + i) * kRowStride), RESET_BOUND);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < N; ++i) next[i * n + e] = q[i];
-#pragma unroll
-  for (int i = 0; i < N; ++i) next[(N + i) * n + e] = v[i];
-}
-
-template <int C>
-__global__ __launch_bounds__(kBlock) void reset_kernel(const float* __restrict__ stand, float* __restrict__ state,
-                                                       uint32_t seed, int64_t n) {
-  constexpr int N = 3 + C;
-  const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (e >= n) return;
-  const uint32_t h = env_hash(seed, (uint32_t)e);
-#pragma unroll
-  for (int i = 0; i < 2 * N; ++i)
-    state[i * n + e] = stand[i] + uniform_pm(pcg_hash(h + (uint32_t)i * kRowStride), RESET_BOUND);
-}
-
-// The hopper's reset (hopper_mlx.py:19-20 with the counter RNG of hopper_metal.py:118-120):
-// the standing pose (0, L, 0, 0, 0, 0, 0, 0) plus U[+-0.05] on every row.
-__global__ __launch_bounds__(kBlock) void hopper_reset_kernel(float* __restrict__ state, uint32_t seed, int64_t n) {
-  const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (e >= n) return;
-  const uint32_t h = env_hash(seed, (uint32_t)e);
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-    state[i * n + e] = (i == 1 ? 1.0f : 0.0f) + uniform_pm(pcg_hash(h + (uint32_t)i * kRowStride), RESET_BOUND);
-}
-
 // Fused ES rollout (legged_rollout_metal.py:19-59). Weight d of member i is
 // theta[i * D + d] (rows) or theta[d * p + i] (columns).
 template <int C, int HID, bool kColumns>
@@ -1251,9 +572,6 @@ constexpr int kTailWaves = C > 2 ? 1 : kTailLanes<C> == 16 ? 2 : LEGGED_SMALL_TA
 // earlier 8-lane groups spilled at C = 2 and were slower than one member per lane).
 template <int C>
 constexpr bool kGroupChunks = true;
-// LDS floats per member for the group substep's Delassus and contact blocks (xd)
-template <int C>
-constexpr int kBlockFloats = 4 * C * C + 12 * C;
 
 // kChunk false: every member runs to the end of its episode. kChunk true: at most chunk_steps
 // steps, then the survivors are appended to dst like rollout_chunk_kernel's (the member's
@@ -2073,14 +1391,6 @@ int dispatch_chunked(bool rows, int32_t hidden, const float* state, const float*
                                                   gate, assist, fitness, steps, workspace, s);
 }
 
-template <int C>
-int launch_step(const float* state, const int32_t* action, uint32_t seed, const float* stand, int iters, double assist,
-                float* next, float* reward, uint8_t* done, int64_t n, hipStream_t s) {
-  hipLaunchKernelGGL(step_kernel<C>, dim3(grid_for(n)), dim3(kBlock), 0, s, state, action, seed, stand, iters,
-                     (float)assist, (float)(0.1 * assist), next, reward, done, n);
-  return launch_status();
-}
-
 template <int C, int HID>
 int launch_rollout(bool columns, const float* state, const float* theta, int64_t p, int32_t horizon, int iters,
                    float alive, float fall, float gate, double assist, float* fitness, float* steps, hipStream_t s) {
@@ -2113,46 +1423,11 @@ int dispatch_hidden(int32_t hidden, bool columns, const float* state, const floa
 
 using namespace hipenvs;
 
-static constexpr int kMaxIters = 4096;
-
-extern "C" int hipenvs_legged_reset(int32_t c, const float* stand, float* state, int64_t n, uint32_t seed,
-                                    hipenvs_stream_t stream) {
-  if (n < 0 || (n > 0 && (!stand || !state))) return HIPENVS_E_ARG;
-  if (n == 0) return HIPENVS_OK;
-  hipStream_t s = as_stream(stream);
-  const dim3 grid(grid_for(n)), block(kBlock);
-  switch (c) {
-    case 1: hipLaunchKernelGGL(lg::reset_kernel<1>, grid, block, 0, s, stand, state, seed, n); break;
-    case 2: hipLaunchKernelGGL(lg::reset_kernel<2>, grid, block, 0, s, stand, state, seed, n); break;
-    case 3: hipLaunchKernelGGL(lg::reset_kernel<3>, grid, block, 0, s, stand, state, seed, n); break;
-    case 4: hipLaunchKernelGGL(lg::reset_kernel<4>, grid, block, 0, s, stand, state, seed, n); break;
-    default: return HIPENVS_E_UNSUPPORTED;
-  }
-  return launch_status();
-}
-
-extern "C" int hipenvs_legged_step(int32_t c, int32_t iters, double assist, const float* state, const int32_t* action,
-                                   uint32_t seed, const float* stand, float* next_state, float* reward, uint8_t* done,
-                                   int64_t n, hipenvs_stream_t stream) {
-  if (n < 0 || iters < 0 || iters > kMaxIters ||
-      (n > 0 && (!state || !action || !stand || !next_state || !reward || !done)))
-    return HIPENVS_E_ARG;
-  if (n == 0) return HIPENVS_OK;
-  hipStream_t s = as_stream(stream);
-  switch (c) {
-    case 1: return lg::launch_step<1>(state, action, seed, stand, iters, assist, next_state, reward, done, n, s);
-    case 2: return lg::launch_step<2>(state, action, seed, stand, iters, assist, next_state, reward, done, n, s);
-    case 3: return lg::launch_step<3>(state, action, seed, stand, iters, assist, next_state, reward, done, n, s);
-    case 4: return lg::launch_step<4>(state, action, seed, stand, iters, assist, next_state, reward, done, n, s);
-    default: return HIPENVS_E_UNSUPPORTED;
-  }
-}
-
 extern "C" int hipenvs_legged_es_rollout(int32_t c, int32_t hidden, int32_t iters, int32_t layout, const float* state,
                                          const float* theta, int64_t p, int32_t horizon, float alive_bonus,
                                          float fall_penalty, float height_gate, double assist, float* fitness,
                                          float* steps, hipenvs_stream_t stream) {
-  if (p < 0 || horizon < 0 || iters < 0 || iters > kMaxIters || (layout != 0 && layout != 1) ||
+  if (p < 0 || horizon < 0 || iters < 0 || iters > lg::kMaxIters || (layout != 0 && layout != 1) ||
       (p > 0 && (!state || !theta || !fitness || !steps)))
     return HIPENVS_E_ARG;
   if (p == 0) return HIPENVS_OK;
@@ -2181,7 +1456,7 @@ int legged_chunked(bool rows, int32_t c, int32_t hidden, int32_t iters, int32_t 
                    const float* theta0, int64_t p, int32_t horizon, float alive_bonus, float fall_penalty,
                    float height_gate, double assist, float* fitness, float* steps, void* workspace,
                    int64_t workspace_bytes, hipenvs_stream_t stream) {
-  if (p < 0 || horizon < 0 || iters < 0 || iters > kMaxIters || chunk_steps < 1 || p > 0x7fffffffLL ||
+  if (p < 0 || horizon < 0 || iters < 0 || iters > lg::kMaxIters || chunk_steps < 1 || p > 0x7fffffffLL ||
       (p > 0 && (!state || !theta0 || !fitness || !steps || !workspace)))
     return HIPENVS_E_ARG;
   if (rows && ((uintptr_t)theta0 & 3u) != 0) return HIPENVS_E_ARG;  // rows are read as dword-aligned vectors
@@ -2231,7 +1506,7 @@ extern "C" int hipenvs_legged_es_rollout_seeded(int32_t c, int32_t hidden, int32
                                                 float fall_penalty, float height_gate, double assist,
                                                 float* fitness, float* steps, void* workspace,
                                                 int64_t workspace_bytes, hipenvs_stream_t stream) {
-  if (p < 2 || (p & 1) || p > 0x7fffffffLL || horizon < 0 || iters < 0 || iters > kMaxIters || chunk_steps < 1 ||
+  if (p < 2 || (p & 1) || p > 0x7fffffffLL || horizon < 0 || iters < 0 || iters > lg::kMaxIters || chunk_steps < 1 ||
       !state || !theta || !fitness || !steps || !workspace)
     return HIPENVS_E_ARG;
   const int64_t need = hipenvs_legged_es_rollout_workspace_bytes(c, hidden, p);
@@ -2255,7 +1530,7 @@ extern "C" int hipenvs_legged_es_rollout_seeded(int32_t c, int32_t hidden, int32
 extern "C" int hipenvs_legged_evaluate(int32_t c, int32_t hidden, int32_t iters, const float* state,
                                        const float* theta, int64_t n, int32_t steps, float eval_bonus,
                                        float* fitness, hipenvs_stream_t stream) {
-  if (n < 0 || steps < 0 || iters < 0 || iters > kMaxIters || (n > 0 && (!state || !theta || !fitness)))
+  if (n < 0 || steps < 0 || iters < 0 || iters > lg::kMaxIters || (n > 0 && (!state || !theta || !fitness)))
     return HIPENVS_E_ARG;
   if (n == 0) return HIPENVS_OK;
   hipStream_t s = as_stream(stream);
@@ -2266,21 +1541,4 @@ extern "C" int hipenvs_legged_evaluate(int32_t c, int32_t hidden, int32_t iters,
     case 4: return lg::launch_evaluate<4>(hidden, state, theta, n, steps, iters, eval_bonus, fitness, s);
     default: return HIPENVS_E_UNSUPPORTED;
   }
-}
-
-extern "C" int hipenvs_hopper_reset(float* state, int64_t n, uint32_t seed, hipenvs_stream_t stream) {
-  if (n < 0 || (n > 0 && !state)) return HIPENVS_E_ARG;
-  if (n == 0) return HIPENVS_OK;
-  hipLaunchKernelGGL(lg::hopper_reset_kernel, dim3(grid_for(n)), dim3(kBlock), 0, as_stream(stream), state, seed, n);
-  return launch_status();
-}
-
-extern "C" int hipenvs_hopper_step(const float* state, const int32_t* action, uint32_t seed, float* next_state,
-                                   float* reward, uint8_t* done, int64_t n, hipenvs_stream_t stream) {
-  if (n < 0 || (n > 0 && (!state || !action || !next_state || !reward || !done))) return HIPENVS_E_ARG;
-  if (n == 0) return HIPENVS_OK;
-  // one exact contact solve per substep: the C = 1 body with one sweep, no assist
-  hipLaunchKernelGGL((lg::step_kernel<1, true>), dim3(grid_for(n)), dim3(kBlock), 0, as_stream(stream), state, action,
-                     seed, nullptr, 1, 0.0f, 0.0f, next_state, reward, done, n);
-  return launch_status();
 }
