@@ -53,6 +53,48 @@ def test_step_at_the_benchmark_size(dev):
     assert 0 < edone.sum() < len(edone)
 
 
+def _rough_states(c, n, seed):
+    """legged_states with members off the ground, deep in it, fast, and with infinite, NaN, huge
+    and tiny positions and velocities: every branch of a contact solve, and its limits."""
+    state, action = legged_states(c, n, seed=seed)
+    r = np.random.default_rng(seed + 1)
+    state[1, r.random(n) < 0.2] += np.float32(2.0)
+    state[1, r.random(n) < 0.2] -= np.float32(1.0)
+    state[3 + c:, r.random(n) < 0.2] *= np.float32(50.0)
+    odd = np.array([np.inf, -np.inf, np.nan, 3e38, -3e38, 1e-42, -1e-42, 0.0, -0.0], np.float32)
+    for col in np.flatnonzero(r.random(n) < 0.3):
+        for row in r.integers(0, 2 * (3 + c), r.integers(1, 4)):
+            state[row, col] = odd[r.integers(len(odd))]
+    return state, action.astype(np.int32)
+
+
+@pytest.mark.parametrize("c", [1, 2, 3, 4])
+@pytest.mark.parametrize("iters,assist", [(0, None), (1, 5.0), (8, None)])
+def test_step_forms_give_the_same_bits(dev, c, iters, assist):
+    """Batches at each bound of the lane-group rule (16 and 64 envs per CU), with ragged last
+    workgroups, against the one-lane kernel (which the tests above pin to the oracle) stepping
+    the same envs in a larger batch: the same state, reward and flag for every env, NaN for
+    NaN."""
+    from hipenvs import legged
+
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    n = 64 * cus + 1
+    state, action = (torch.from_numpy(x).to(dev) for x in _rough_states(c, n, seed=30 + c))
+    body = legged.Legged(c, iters)
+
+    def step(m):
+        body.reseed(9)
+        return [to_np(t) for t in body.step(state[:, :m].contiguous(), action[:m], assist)]
+
+    whole = step(n)  # past 64 per CU: one lane per env
+    for m in (1, 3, 17, 16 * cus, 16 * cus + 1, 64 * cus):
+        for got, want in zip(step(m), whole):
+            np.testing.assert_array_equal(got, want[..., :m])
+            zeros = want[..., :m] == 0  # and the sign of a zero
+            np.testing.assert_array_equal(np.signbit(got[zeros].astype(np.float32)),
+                                          np.signbit(want[..., :m][zeros].astype(np.float32)))
+
+
 @pytest.mark.parametrize("c", [2, 4])
 def test_step_with_assist_matches_oracle(dev, c):
     from hipenvs import legged
