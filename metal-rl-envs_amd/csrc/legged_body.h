@@ -85,6 +85,25 @@ __device__ __forceinline__ ContactBlock contact_block(float Att, float Atn, floa
   return b;
 }
 
+// What a contact's depth fixes for all sweeps of a substep, for the lane groups: target =
+// 20 max(depth, 0), and `closed`, which target - wn must exceed for the contact to push: 0, or
+// +inf off the ground. That is touching && wn < target as one compare of the difference, whose
+// sign is exact (no difference of two unequal floats rounds to 0). Shut, a contact may not stick
+// (the sweep makes its cone NaN wide) and its edges are 0 by themselves: their numerator is 0.
+struct ContactGate {
+  float target, closed;
+};
+
+// The contact's gate. A cone edge has no impulse when its denominator is not positive or the
+// foot is off the ground: its reciprocal becomes -2^-300, so that the quotient of its numerator
+// (target - wn or 0) is -0 or -inf, or all is NaN, and the sweep's clamp at 0 needs no mask.
+__device__ __forceinline__ ContactGate contact_gate(ContactBlock& b, float depth) {
+  const bool touching = depth >= 0.0f;
+  b.rden_p = (b.den_p > 0.0f && touching) ? b.rden_p : -0x1p-300;
+  b.rden_m = (b.den_m > 0.0f && touching) ? b.rden_m : -0x1p-300;
+  return ContactGate{BAUMGARTE_OVER_H * max0(depth), touching ? 0.0f : __builtin_inff()};
+}
+
 template <class Div>
 __device__ __forceinline__ void contact_impulse(const ContactBlock& b, float wt, float wn, float depth,
                                                 float& lt_out, float& ln_out, Div& div) {
@@ -132,13 +151,13 @@ __device__ __forceinline__ void chol_solve(const float (&L)[N][N], const double 
   }
 }
 
-// sa[k], ca[k] = lane k's sn, cs, for k < K, on every lane of the G-lane group.
-template <int G, int K>
+// sa[k], ca[k] = lane k * kStride's sn, cs, for k < K, on every lane of the G-lane group.
+template <int G, int K, int kStride>
 __device__ __forceinline__ void row_trig(float sn, float cs, float* sa, float* ca) {
   if constexpr (K > 0) {
-    row_trig<G, K - 1>(sn, cs, sa, ca);
-    sa[K - 1] = lane_bcast<G, K - 1>(sn);
-    ca[K - 1] = lane_bcast<G, K - 1>(cs);
+    row_trig<G, K - 1, kStride>(sn, cs, sa, ca);
+    sa[K - 1] = lane_bcast<G, (K - 1) * kStride>(sn);
+    ca[K - 1] = lane_bcast<G, (K - 1) * kStride>(cs);
   }
 }
 
@@ -156,16 +175,16 @@ template <int C>
 constexpr int kBlockFloats = 4 * C * C + 12 * C;
 
 // One semi-implicit Euler substep with block PGS contacts, in place (legged_np.py:57-97).
-// kGroup = 0: one lane computes the whole substep. kGroup = G (8 or 16): the G lanes
-// g = 0..G-1 of a member's group (a 16-lane DPP row or half of one) all hold the member's
-// state and compute everything identically, except that lane g < C evaluates foot g's sin
-// and cos, shared by DPP broadcast, the Gauss-Seidel sweeps and the velocity update split
-// their independent work over the lanes (below), and lane g solves right-hand sides g,
-// g + G, ... of the 2C + 1 triangular solves
-// (the forces, then the tangent, then the normal Jacobian rows), exchanged through the
-// group's LDS rows xs ((2C + 1) x 8 floats). Every value is computed by the same expression
-// as in the one-lane form, so the results are the same bits. Callers keep the group's
-// lanes in one single-wave workgroup, so the barriers order its LDS traffic.
+// kGroup = 0: one lane computes the whole substep. kGroup = G (4, 8 or 16): the G lanes
+// g = 0..G-1 of a member's group (a DPP quad, a 16-lane DPP row or half of one) all hold the
+// member's state and compute everything identically, except that the lanes share by DPP
+// broadcast the feet's sines and cosines, one foot a lane, split the 2C + 1 triangular solves
+// (the forces and the Jacobian's columns), the C^2 Delassus blocks, the Gauss-Seidel sweeps and
+// the velocity update between them (below), and exchange the solves through the group's LDS
+// rows xs ((2C + 1) x 8 floats: forces, tangent columns, normal columns) and the blocks through
+// xd. Every value is computed by the same expression as in the one-lane form, so the results
+// are the same bits. Callers keep the group's lanes in one single-wave workgroup, so the
+// barriers order its LDS traffic.
 // kHopperSum (C = 1 only) adds the impulse terms as the reference's hopper does,
 // (v_free + M^-1 J_t^T lt) + M^-1 J_n^T ln (hopper_np.py:76), instead of the legged body's
 // v_free + (M^-1 J_t^T lt + M^-1 J_n^T ln) (legged_np.py:95); otherwise the hopper is this
@@ -179,15 +198,23 @@ __device__ __forceinline__ void substep(float (&q)[3 + C], float (&v)[3 + C], co
                                         int g = 0, float* xd = nullptr) {
   constexpr int N = 3 + C;
   float ca[C], sa[C], dx[C], dy[C], depth[C], r2[C];
+  // kRows: every lane has a coupling row of its own, row g % 2C (contact g % 2C / 2, tangential or
+  // normal as g is even or odd), and evaluates its contact's sin and cos: its right-hand side,
+  // its Delassus blocks, its gate and its free velocity then need no selection among the feet:
+  // 885 -> 790 instructions a substep beside the sweeps (16 lanes, C = 4), quadruped step at
+  // N = 2,048 21.1 -> 20.0 us.
+  constexpr bool kRows = kGroup >= 2 * C && 2 * (kGroup / (2 * C)) >= C;
+  const int krow = kRows ? g % (2 * C) : 0, kown = krow / 2;
+  const bool nown = krow % 2 != 0;
+  float sn = 0.0f, cs = 0.0f;  // of the lane's own foot
   if constexpr (kGroup >= 4 && kGroup >= C) {
-    // lane g < C evaluates foot g's sin and cos, shared by DPP broadcast within the group
+    // shared by DPP broadcast within the group, from lane 2k or (not kRows) lane k
     static_assert(C <= kGroup, "one lane per foot");
     float a = q[2] + q[3];
 #pragma unroll
-    for (int k = 1; k < C; ++k) a = (g == k) ? q[2] + q[3 + k] : a;
-    float sn, cs;
+    for (int k = 1; k < C; ++k) a = ((kRows ? kown : g) == k) ? q[2] + q[3 + k] : a;
     det_sincos(a, &sn, &cs);
-    row_trig<kGroup, C>(sn, cs, sa, ca);
+    row_trig<kGroup, C, kRows ? 2 : 1>(sn, cs, sa, ca);
   } else {
 #pragma unroll
     for (int k = 0; k < C; ++k) det_sincos(q[2] + q[3 + k], &sa[k], &ca[k]);
@@ -276,31 +303,48 @@ __device__ __forceinline__ void substep(float (&q)[3 + C], float (&v)[3 + C], co
     float b[kRounds][N];
 #pragma unroll
     for (int r = 0; r < kRounds; ++r) {
-      // lane g solves right-hand sides g, g + kGroup, ...; past 2C it solves the forces again, unused
-      const int rhs = g + r * kGroup < kRhs ? g + r * kGroup : 0;
-      const bool normal = rhs > C;
-      const int k = normal ? rhs - 1 - C : rhs - 1;
-      float ck = ca[0], sk = sa[0];
+      if constexpr (kRows) {
+        // the lane's own row's column in the first round; the forces on the lanes past 2C, or
+        // on all of them in a second round when there are none
+        const bool force = g + r * kGroup >= 2 * C;
+        const float c = nown ? sn : cs;
 #pragma unroll
-      for (int kk = 1; kk < C; ++kk) {
-        ck = (k == kk) ? ca[kk] : ck;
-        sk = (k == kk) ? sa[kk] : sk;
-      }
+        for (int i = 0; i < N; ++i) {
+          const float j = (i == 0) ? (nown ? 0.0f : 1.0f)
+                          : (i == 1) ? (nown ? 1.0f : 0.0f)
+                          : (i == 2) ? c : (kown == i - 3) ? c : 0.0f;
+          b[r][i] = force ? f[i] : j;
+        }
+      } else {
+        // lane g solves right-hand sides g, g + kGroup, ...; past 2C it solves the forces again, unused
+        const int rhs = g + r * kGroup < kRhs ? g + r * kGroup : 0;
+        const bool normal = rhs > C;
+        const int k = normal ? rhs - 1 - C : rhs - 1;
+        float ck = ca[0], sk = sa[0];
 #pragma unroll
-      for (int i = 0; i < N; ++i) {
-        const bool on = (i == 2 || i == 3 + k);
-        const float jt = (i == 0) ? 1.0f : on ? ck : 0.0f;
-        const float jn = (i == 1) ? 1.0f : on ? sk : 0.0f;
-        b[r][i] = (rhs == 0) ? f[i] : normal ? jn : jt;
+        for (int kk = 1; kk < C; ++kk) {
+          ck = (k == kk) ? ca[kk] : ck;
+          sk = (k == kk) ? sa[kk] : sk;
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          const bool on = (i == 2 || i == 3 + k);
+          const float jt = (i == 0) ? 1.0f : on ? ck : 0.0f;
+          const float jn = (i == 1) ? 1.0f : on ? sk : 0.0f;
+          b[r][i] = (rhs == 0) ? f[i] : normal ? jn : jt;
+        }
       }
       chol_solve<N>(L, rL, b[r], div);
     }
     __syncthreads();  // the rows' previous readers are done
 #pragma unroll
     for (int r = 0; r < kRounds; ++r) {
-      if (g + r * kGroup < kRhs) {
+      const int h = g + r * kGroup;
+      if (h < kRhs) {
+        // rows of xs: the forces, the tangent columns, the normal columns
+        const int row = !kRows ? h : h == 2 * C ? 0 : 1 + h / 2 + (h % 2) * C;
 #pragma unroll
-        for (int i = 0; i < N; ++i) xs[(g + r * kGroup) * kRow + i] = b[r][i];
+        for (int i = 0; i < N; ++i) xs[row * kRow + i] = b[r][i];
       }
     }
     __syncthreads();
@@ -318,30 +362,47 @@ __device__ __forceinline__ void substep(float (&q)[3 + C], float (&v)[3 + C], co
     // diagonal block also forms its contact's ContactBlock; the group reads the C^2 blocks
     // (4 floats each) and the C contact blocks (12 floats each) back from xd
     constexpr int kRow = 8;
-    constexpr int kBlocks = C * C, kRounds = (kBlocks + kGroup - 1) / kGroup;
+    constexpr int kBlocks = C * C, kRounds = kRows ? 1 : (kBlocks + kGroup - 1) / kGroup;
 #pragma unroll
     for (int r = 0; r < kRounds; ++r) {
-      const int gr = g + r * kGroup;
-      const int gb = gr < kBlocks ? gr : 0;  // lanes past C^2 form block 0 again, unused
-      const int kb = gb / C, lb = gb % C;
-      float ck = ca[0], sk = sa[0];
+      int kb, lb;
+      bool mine;
+      float ck, sk;
+      if constexpr (kRows) {  // row kown's blocks, 2 to each set of 2C lanes
+        kb = kown;
+        lb = 2 * (g / (2 * C)) + g % 2;
+        mine = lb < C;
+        lb = mine ? lb : 0;
+        ck = cs;
+        sk = sn;
+      } else {
+        const int gr = g + r * kGroup;
+        mine = gr < kBlocks;
+        const int gb = mine ? gr : 0;  // lanes past C^2 form block 0 again, unused
+        kb = gb / C;
+        lb = gb % C;
+        ck = ca[0];
+        sk = sa[0];
 #pragma unroll
-      for (int kk = 1; kk < C; ++kk) {
-        ck = (kb == kk) ? ca[kk] : ck;
-        sk = (kb == kk) ? sa[kk] : sk;
+        for (int kk = 1; kk < C; ++kk) {
+          ck = (kb == kk) ? ca[kk] : ck;
+          sk = (kb == kk) ? sa[kk] : sk;
+        }
       }
       const float* rt = xs + (1 + lb) * kRow;
       const float* rn = xs + (1 + C + lb) * kRow;
       const float t2 = rt[2], t3 = rt[3 + kb], n2 = rn[2], n3 = rn[3 + kb];
       const float4 blk4 = make_float4((rt[0] + ck * t2) + ck * t3, (rn[0] + ck * n2) + ck * n3,
                                       (rt[1] + sk * t2) + sk * t3, (rn[1] + sk * n2) + sk * n3);
-      if (gr < kBlocks) *reinterpret_cast<float4*>(xd + 4 * gr) = blk4;
-      const ContactBlock own = contact_block(blk4.x, blk4.y, blk4.w);
-      if (gr < kBlocks && kb == lb) {
+      if (mine) *reinterpret_cast<float4*>(xd + 4 * (kb * C + lb)) = blk4;
+      ContactBlock own = contact_block(blk4.x, blk4.y, blk4.w);
+      if (mine && kb == lb) {
+        const ContactGate gate = contact_gate(own, -(q[1] - ck));
         float* xc = xd + 4 * C * C + 12 * kb;
-        *reinterpret_cast<float4*>(xc) = make_float4(own.det, own.den_p, own.den_m, 0.0f);
+        *reinterpret_cast<float4*>(xc) = make_float4(own.det, own.den_p, own.den_m, own.Att * MU + own.Atn);
         *reinterpret_cast<double2*>(xc + 4) = make_double2(own.rdet, own.rden_p);
         *reinterpret_cast<double*>(xc + 8) = own.rden_m;
+        *reinterpret_cast<float2*>(xc + 10) = make_float2(gate.target, gate.closed);
       }
     }
     __syncthreads();
@@ -368,10 +429,19 @@ __device__ __forceinline__ void substep(float (&q)[3 + C], float (&v)[3 + C], co
       }
     }
   }
+  float w0own = 0.0f;
+  if constexpr (kRows) {
+    const float c = nown ? sn : cs;
+    float vk = vf[3];
 #pragma unroll
-  for (int k = 0; k < C; ++k) {
-    w0t[k] = (vf[0] + ca[k] * vf[2]) + ca[k] * vf[3 + k];
-    w0n[k] = (vf[1] + sa[k] * vf[2]) + sa[k] * vf[3 + k];
+    for (int k = 1; k < C; ++k) vk = (kown == k) ? vf[3 + k] : vk;
+    w0own = ((nown ? vf[1] : vf[0]) + c * vf[2]) + c * vk;
+  } else {
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+      w0t[k] = (vf[0] + ca[k] * vf[2]) + ca[k] * vf[3 + k];
+      w0n[k] = (vf[1] + sa[k] * vf[2]) + sa[k] * vf[3 + k];
+    }
   }
   if constexpr (kStage) {
     static_assert(kGroup == 0, "staging is for the one-lane form");
@@ -392,15 +462,7 @@ __device__ __forceinline__ void substep(float (&q)[3 + C], float (&v)[3 + C], co
   for (int k = 0; k < C; ++k) {
     lt[k] = 0.0f;
     ln[k] = 0.0f;
-    if constexpr (kGroup > 0) {
-      const float* xc = xd + 4 * C * C + 12 * k;
-      const float4 f4 = *reinterpret_cast<const float4*>(xc);
-      const double2 d2 = *reinterpret_cast<const double2*>(xc + 4);
-      blk[k] = ContactBlock{Att[k][k], Atn[k][k], Ann[k][k], f4.x, f4.y, f4.z,
-                            d2.x, d2.y, *reinterpret_cast<const double*>(xc + 8)};
-    } else {
-      blk[k] = contact_block(Att[k][k], Atn[k][k], Ann[k][k]);
-    }
+    if constexpr (kGroup == 0) blk[k] = contact_block(Att[k][k], Atn[k][k], Ann[k][k]);
   }
   if constexpr (kGroup >= 4) {
     // The member's lanes split the sweep's independent work and share the results by DPP
@@ -414,8 +476,9 @@ __device__ __forceinline__ void substep(float (&q)[3 + C], float (&v)[3 + C], co
     // sweep evaluates, so the impulses are the same bits.
     // Each lane reads its own coefficients from the group's LDS blocks at a lane-dependent
     // offset (block (k, l) holds Att, Atn, Ant, Ann; contact k's block holds det, den_p,
-    // den_m and then their float64 reciprocals), and negates by flipping the sign bit: no
-    // per-lane selects, which the compiler had turned into exec-mask branches.
+    // den_m, the slope of slip and then the three's float64 reciprocals, target and closed), and
+    // negates by flipping the sign bit: no per-lane selects, which the compiler had turned into
+    // exec-mask branches.
     constexpr int kSlots = (2 * C + kGroup - 1) / kGroup;
     const int sel = (g == 2) ? 1 : (g == 3) ? 2 : 0;       // det, den_p, den_m
     const uint32_t neg = (g == 1) ? 0x80000000u : 0u;
@@ -424,10 +487,11 @@ __device__ __forceinline__ void substep(float (&q)[3 + C], float (&v)[3 + C], co
     // so: no mask on the chain is combined on the scalar unit, which would wait for the vector
     // compare to complete (the gate is one compare before the quotients and works through the
     // cone's width); broadcasts fold into their uses (v_sub, v_mul, v_add, v_max with a DPP
-    // operand). 16 lanes, C = 4: 163 instructions a sweep (145 VALU) where per-pair coupling
+    // operand). 16 lanes, C = 4: about 164 instructions a sweep (145 VALU) where per-pair coupling
     // terms, separate broadcasts and a masked clamp and gate took 203 (182 VALU). Quadruped ES
     // rollout at P = 262,144, H = 64, 1,000 steps, 8 sweeps 30.6 -> 27.1 ms; generation at
-    // P = 1,024, H = 16, every member standing for 500 steps 20.2 -> 17.5 ms.
+    // P = 1,024, H = 16, every member standing for 500 steps 20.2 -> 17.5 ms (17.05 with a row of the
+    // setup per lane too, kRows).
     const bool edge = (g == 2 || g == 3);
     float cA[kSlots][C], cB[kSlots][C], w0x[kSlots], t[kSlots][C];
     float qP[C], qQ[C], qd[C], slipc[C], target[C], closed[C];
@@ -437,9 +501,11 @@ __device__ __forceinline__ void substep(float (&q)[3 + C], float (&v)[3 + C], co
     for (int s = 0; s < kSlots; ++s) {
       const int row = (s * kGroup + g) % (2 * C);  // lanes past 2C repeat the rows from the first
       const float* xr = xd + 4 * C * (row / 2) + 2 * (row % 2);     // Att, Atn or Ant, Ann of contact row / 2
-      w0x[s] = w0t[0];
+      w0x[s] = kRows ? w0own : w0t[0];
+      if constexpr (!kRows) {
 #pragma unroll
-      for (int r = 1; r < 2 * C; ++r) w0x[s] = (row == r) ? (r % 2 ? w0n[r / 2] : w0t[r / 2]) : w0x[s];
+        for (int r = 1; r < 2 * C; ++r) w0x[s] = (row == r) ? (r % 2 ? w0n[r / 2] : w0t[r / 2]) : w0x[s];
+      }
 #pragma unroll
       for (int l = 0; l < C; ++l) {
         cA[s][l] = xr[4 * l];
@@ -458,22 +524,14 @@ __device__ __forceinline__ void substep(float (&q)[3 + C], float (&v)[3 + C], co
       const float* xc = xd + 4 * C * C + 12 * k;
       qd[k] = xc[sel];
       qr[k] = *reinterpret_cast<const double*>(xc + 4 + 2 * sel);
-      // A cone edge has no impulse when its denominator is not positive or the foot is off the
-      // ground: its lane multiplies by -2^-300 instead, so the quotient of its numerator
-      // (target - wn or 0) is -0 or -inf, and the clamp at 0 below needs no mask. The sign of
-      // a zero edge impulse reaches no result: it is added to wt for a comparison with 0, and
-      // it is not positive.
-      const bool touching = depth[k] >= 0.0f;
-      qzero[k] = edge && !(qd[k] > 0.0f && touching);  // lane 2 holds den_p, lane 3 den_m
-      qr[k] = qzero[k] ? -0x1p-300 : qr[k];
-      slipc[k] = blk[k].Att * MU + blk[k].Atn;
-      // A contact pushes only if touching && wn < target, which is one compare of target - wn
-      // (whose sign is exact: no difference of two unequal floats rounds to 0) with 0, or with
-      // +inf off the ground. Shut, it may not stick (the cone is NaN wide), and its edges are
-      // 0 by themselves: their numerator is 0, or the line above, or all is NaN and nothing
-      // is positive.
-      target[k] = BAUMGARTE_OVER_H * max0(depth[k]);
-      closed[k] = touching ? 0.0f : __builtin_inff();
+      // lane 2 holds den_p, lane 3 den_m; an edge that has no impulse a negative reciprocal
+      // (contact_gate). The sign of a zero edge impulse reaches no result: it is added to wt
+      // for a comparison with 0, and it is not positive.
+      qzero[k] = !Div::kRecip && edge && qr[k] < 0.0;
+      const float2 gate = *reinterpret_cast<const float2*>(xc + 10);
+      target[k] = gate.x;
+      closed[k] = gate.y;
+      slipc[k] = xc[3];
     }
     // in vector registers: 0, so that the clamps fold their broadcasts, and the edge lanes as
     // bits, so that the loop selects by them (on a condition the compiler knows to be
