@@ -522,24 +522,24 @@ constexpr int kTile = 64;
 
 __host__ __device__ constexpr int64_t round_to_tile(int64_t n) { return (n + kTile - 1) / kTile * kTile; }
 
-// The tail of a rollout: once at most wide_max members survive (about one wave per SIMD in
-// this form), each compacted member gets a group of kTailLanes<C> lanes and runs to the end
-// of its episode (policy_group, substep_exact_group), kTailMembers<C> members per wave. The
-// group shortens one member's step, which is what bounds the tail. Results are those of the
-// one-lane schedule, bit for bit.
-// At C <= 2 every lane role fits in 8 lanes (2C + 1 solves, C^2 Delassus blocks, 3C heads),
-// so eight members share a wave and the tail runs one wave per SIMD from 32 survivors per CU.
-// With 16 lanes it ran two 4-member waves per SIMD from the same count, which share the
-// SIMD's issue to the end of the horizon: biped ES rollout at N = 262,144 19.6 -> 17.9,
-// 23.8 -> 21.7 and 32.4 -> 30.2 ms at 4, 8 and 16 sweeps. Eight lanes at two waves per SIMD
-// from 64 per CU (LEGGED_SMALL_TAIL_WAVES 2, no group chunks) took 20.6, 25.5 and 35.2 ms.
-#ifndef LEGGED_SMALL_TAIL_LANES
-#define LEGGED_SMALL_TAIL_LANES 8
-#endif
+// The tail of a rollout: once at most wide_max members survive (one wave per SIMD in this
+// form), each compacted member gets a group of 16 lanes and runs to the end of its episode
+// (policy_group, substep_exact_group), four members to a wave. The group shortens one member's
+// step, which is what bounds the tail. Results are those of the one-lane schedule, bit for bit.
+// At C <= 2 every lane role also fits in 8 lanes (2C + 1 solves, C^2 Delassus blocks, 3C
+// heads), eight members to a wave. A step is longer that way (two moves a broadcast, twice the
+// hidden units a lane), but one launch holds twice the members: it runs populations of 16 to 32
+// members per CU, which then need no chunks. H = 32, 300 steps, 8 sweeps, ms (8 lanes / 16):
+//   biped, P = 4,096 standing 3.50 / 3.06, falling 3.42 / 3.08; P = 8,192 standing 3.51 / 4.36,
+//   falling 3.49 / 3.23; P = 65,536 falling 4.54 / 4.20; H = 64, P = 262,144 7.10 / 6.67
+//   one leg, P = 4,096 0.65 / 0.58; P = 262,144 3.66 / 3.60
+constexpr int kTailLanes = 16, kSmallTailLanes = 8;
+constexpr int64_t kTailPerCu = 4 * (64 / kTailLanes), kSmallTailPerCu = 4 * (64 / kSmallTailLanes);
+// Whether n members or envs on `cus` CUs take the 8-lane form.
 template <int C>
-constexpr int kTailLanes = C <= 2 ? LEGGED_SMALL_TAIL_LANES : 16;
-template <int C>
-constexpr int kTailMembers = 64 / kTailLanes<C>;
+inline bool small_tail(int64_t n, int cus) {
+  return C <= 2 && n > kTailPerCu * cus && n <= kSmallTailPerCu * cus;
+}
 // Above the tail's bound and up to this many survivors per CU, a chunk runs in the group form
 // (rollout_group_chunk_kernel) instead of one member per lane, with LEGGED_GROUP_CHUNK_LANES
 // lanes per member. With the split Gauss-Seidel sweeps (a 4-lane group broadcasts with one
@@ -554,22 +554,9 @@ constexpr int kTailMembers = 64 / kTailLanes<C>;
 #define LEGGED_GROUP_CHUNK_LANES 4
 #endif
 constexpr int kChunkGroupLanes = LEGGED_GROUP_CHUNK_LANES;
-// Waves per SIMD the group tail runs at; it takes over at 4 x kTailWaves x kTailMembers
-// survivors per CU. With its members' weights in registers the 16-lane form needed 218 VGPRs
-// at C = 2 (H = 64), so two waves shared a SIMD; at C = 4 it needs 256 VGPRs + 14 AGPRs, one
-// wave per SIMD. (Reloading the weights every step instead fits two waves at C = 4, 206 VGPRs,
-// but the ES rollout at N = 262,144 and 8 sweeps took 60.6 instead of 50.0 ms: a SIMD holding
-// two long-lived members' waves steps each at part speed to the end of the horizon.)
-#ifndef LEGGED_SMALL_TAIL_WAVES
-#define LEGGED_SMALL_TAIL_WAVES 1
-#endif
-template <int C>
-constexpr int kTailWaves = C > 2 ? 1 : kTailLanes<C> == 16 ? 2 : LEGGED_SMALL_TAIL_WAVES;
 // Whether chunks between the tail's bound and LEGGED_GROUP_CHUNK_MEMBERS_PER_CU run in the
-// group form. At C <= 2 the tail already takes over at 32 per CU; with 4-lane groups at one
-// wave per SIMD the biped's group chunks between 32 and 64 per CU also pay (biped ES rollout
-// at N = 262,144: 20.2 -> 19.7, 24.9 -> 24.1 and 35.2 -> 33.0 ms at 4, 8, 16 sweeps; the
-// earlier 8-lane groups spilled at C = 2 and were slower than one member per lane).
+// group form. (Biped ES rollout at N = 262,144 with the tail from 32 per CU: group chunks
+// between 32 and 64 per CU 20.2 -> 19.7, 24.9 -> 24.1 and 35.2 -> 33.0 ms at 4, 8, 16 sweeps.)
 template <int C>
 constexpr bool kGroupChunks = true;
 
@@ -680,31 +667,31 @@ __device__ __forceinline__ void rollout_group(const Packed& src, const Packed& d
 // The group tail as a kernel of its own, launched after every later chunk: it runs when the
 // set holds at most wide_max members and exits at once otherwise (the chunk kernels do the
 // opposite). Kept apart so that the one-lane kernel's code is compiled on its own.
-template <int C, int HID>
-__global__ __launch_bounds__(64, kTailWaves<C>) void rollout_tail_kernel(Packed src, int64_t cap, int32_t horizon, int iters,
+template <int C, int HID, int G>
+__global__ __launch_bounds__(64, 1) void rollout_tail_kernel(Packed src, int64_t cap, int32_t horizon, int iters,
                                                           float alive_bonus, float fall, float gate, float assist,
                                                           float assist_damping, float* __restrict__ fitness,
                                                           float* __restrict__ steps_out, int64_t wide_max) {
   const int64_t count = (int64_t)*src.count;
   if (count > wide_max) return;
-  LEGGED_GROUP_LDS(C, HID, kTailMembers<C>);
-  rollout_group<C, HID, kTailLanes<C>, false>(src, src, count, cap, horizon, horizon, iters, alive_bonus, fall, gate,
+  LEGGED_GROUP_LDS(C, HID, 64 / G);
+  rollout_group<C, HID, G, false>(src, src, count, cap, horizon, horizon, iters, alive_bonus, fall, gate,
                                             assist, assist_damping, fitness, steps_out, xs_all, xh_all, xl_all,
                                             xd_all);
 }
 
-// The greedy evaluation (evaluate_kernel) with a group of kTailLanes<C> lanes per env, for
+// The greedy evaluation (evaluate_kernel) with the tail's group of G lanes per env, for
 // batches of at most one wave per SIMD: one env per lane leaves most SIMDs idle there, and a
 // policy that stands steps every env to the end at one lane's latency. The shared policy's
 // weights are loaded into the group's registers once; the step is the group tail's (same
 // bits as the one-lane kernel).
-template <int C, int HID>
-__global__ __launch_bounds__(64, kTailWaves<C>) void evaluate_group_kernel(const float* __restrict__ state,
+template <int C, int HID, int G>
+__global__ __launch_bounds__(64, 1) void evaluate_group_kernel(const float* __restrict__ state,
                                                                           const float* __restrict__ theta,
                                                                           int64_t n, int32_t steps, int iters,
                                                                           float eval_bonus,
                                                                           float* __restrict__ fitness) {
-  constexpr int N = 3 + C, OBS = 5 + 2 * C, OUT = 3 * C, G = kTailLanes<C>, M = kTailMembers<C>;
+  constexpr int N = 3 + C, OBS = 5 + 2 * C, OUT = 3 * C, M = 64 / G;
   LEGGED_GROUP_LDS(C, HID, M);
   const int g = (int)threadIdx.x % G, mloc = (int)threadIdx.x / G;
   float* xs = xs_all + mloc * (2 * C + 1) * 8;
@@ -1148,12 +1135,14 @@ __global__ __launch_bounds__(64, LEGGED_FIRST_CHUNK_MIN_WAVES) void rollout_pair
 // the group chunk kernel above wide_max, the group tail at or below wide_max.
 struct GroupBounds {
   int64_t wide_max, group_max, group_grid, tail_grid;
+  bool small_tail;  // the tail runs 8 lanes per member
 };
 
 template <int C>
 inline GroupBounds group_bounds(int64_t p, int cus) {
   GroupBounds b;
-  b.wide_max = (int64_t)4 * kTailWaves<C> * kTailMembers<C> * cus;
+  b.small_tail = small_tail<C>(p, cus);
+  b.wide_max = (b.small_tail ? kSmallTailPerCu : kTailPerCu) * cus;
   const int64_t gm = kGroupChunks<C> ? (int64_t)LEGGED_GROUP_CHUNK_MEMBERS_PER_CU * cus : 0;
   b.group_max = gm > b.wide_max ? gm : b.wide_max;
   // one member group per workgroup: a kernel never holds more than min(p, its bound) members
@@ -1161,7 +1150,8 @@ inline GroupBounds group_bounds(int64_t p, int cus) {
   const int64_t tail_members = p < b.wide_max ? p : b.wide_max;
   constexpr int chunk_members = 64 / kChunkGroupLanes;  // per single-wave workgroup
   b.group_grid = (group_members + chunk_members - 1) / chunk_members;
-  b.tail_grid = (tail_members + kTailMembers<C> - 1) / kTailMembers<C>;
+  const int tail_wave = 64 / (b.small_tail ? kSmallTailLanes : kTailLanes);
+  b.tail_grid = (tail_members + tail_wave - 1) / tail_wave;
   return b;
 }
 
@@ -1182,8 +1172,16 @@ int launch_later_chunk(const float* state0, const float* theta0, int64_t p, cons
                          s, src, dst, cap, chunk_steps, horizon, iters, alive, fall, gate, af, ad, fitness, steps,
                          gb.wide_max, gb.group_max);
   }
-  hipLaunchKernelGGL((rollout_tail_kernel<C, HID>), dim3((unsigned)gb.tail_grid), dim3(64), 0, s, src, cap, horizon,
-                     iters, alive, fall, gate, af, ad, fitness, steps, gb.wide_max);
+  const dim3 tail((unsigned)gb.tail_grid), wave(64);
+  if constexpr (C <= 2) {
+    if (gb.small_tail) {
+      hipLaunchKernelGGL((rollout_tail_kernel<C, HID, kSmallTailLanes>), tail, wave, 0, s, src, cap, horizon, iters,
+                         alive, fall, gate, af, ad, fitness, steps, gb.wide_max);
+      return launch_status();
+    }
+  }
+  hipLaunchKernelGGL((rollout_tail_kernel<C, HID, kTailLanes>), tail, wave, 0, s, src, cap, horizon, iters, alive,
+                     fall, gate, af, ad, fitness, steps, gb.wide_max);
   return launch_status();
 }
 
@@ -1334,6 +1332,21 @@ int dispatch_chunked_seeded(int32_t hidden, const float* state, const float* the
 #ifndef LEGGED_EVALUATE_GROUP
 #define LEGGED_EVALUATE_GROUP 1
 #endif
+template <int C, int G>
+int launch_evaluate_group(int32_t hidden, const float* state, const float* theta, int64_t n, int32_t steps, int iters,
+                          float eval_bonus, float* fitness, hipStream_t s) {
+  const dim3 grid(grid_for(n, 64 / G)), block(64);
+  switch (hidden) {
+    case 4: hipLaunchKernelGGL((evaluate_group_kernel<C, 4, G>), grid, block, 0, s, state, theta, n, steps, iters, eval_bonus, fitness); break;
+    case 8: hipLaunchKernelGGL((evaluate_group_kernel<C, 8, G>), grid, block, 0, s, state, theta, n, steps, iters, eval_bonus, fitness); break;
+    case 16: hipLaunchKernelGGL((evaluate_group_kernel<C, 16, G>), grid, block, 0, s, state, theta, n, steps, iters, eval_bonus, fitness); break;
+    case 32: hipLaunchKernelGGL((evaluate_group_kernel<C, 32, G>), grid, block, 0, s, state, theta, n, steps, iters, eval_bonus, fitness); break;
+    case 64: hipLaunchKernelGGL((evaluate_group_kernel<C, 64, G>), grid, block, 0, s, state, theta, n, steps, iters, eval_bonus, fitness); break;
+    default: return HIPENVS_E_UNSUPPORTED;
+  }
+  return launch_status();
+}
+
 template <int C>
 int launch_evaluate(int32_t hidden, const float* state, const float* theta, int64_t n, int32_t steps, int iters,
                     float eval_bonus, float* fitness, hipStream_t s) {
@@ -1343,17 +1356,13 @@ int launch_evaluate(int32_t hidden, const float* state, const float* theta, int6
   if (query != HIPENVS_OK) return query;
   // a batch that the group form holds at one wave per SIMD takes it (one lane per env would
   // leave most SIMDs idle and step each env at one lane's latency)
-  if (LEGGED_EVALUATE_GROUP && n <= (int64_t)4 * kTailWaves<C> * kTailMembers<C> * cus) {
-    const dim3 ggrid((unsigned)((n + kTailMembers<C> - 1) / kTailMembers<C>));
-    switch (hidden) {
-      case 4: hipLaunchKernelGGL((evaluate_group_kernel<C, 4>), ggrid, block, 0, s, state, theta, n, steps, iters, eval_bonus, fitness); break;
-      case 8: hipLaunchKernelGGL((evaluate_group_kernel<C, 8>), ggrid, block, 0, s, state, theta, n, steps, iters, eval_bonus, fitness); break;
-      case 16: hipLaunchKernelGGL((evaluate_group_kernel<C, 16>), ggrid, block, 0, s, state, theta, n, steps, iters, eval_bonus, fitness); break;
-      case 32: hipLaunchKernelGGL((evaluate_group_kernel<C, 32>), ggrid, block, 0, s, state, theta, n, steps, iters, eval_bonus, fitness); break;
-      case 64: hipLaunchKernelGGL((evaluate_group_kernel<C, 64>), ggrid, block, 0, s, state, theta, n, steps, iters, eval_bonus, fitness); break;
-      default: return HIPENVS_E_UNSUPPORTED;
+  if (LEGGED_EVALUATE_GROUP) {
+    if (n <= kTailPerCu * cus)
+      return launch_evaluate_group<C, kTailLanes>(hidden, state, theta, n, steps, iters, eval_bonus, fitness, s);
+    if constexpr (C <= 2) {
+      if (small_tail<C>(n, cus))
+        return launch_evaluate_group<C, kSmallTailLanes>(hidden, state, theta, n, steps, iters, eval_bonus, fitness, s);
     }
-    return launch_status();
   }
   switch (hidden) {
     case 4: hipLaunchKernelGGL((evaluate_kernel<C, 4>), grid, block, 0, s, state, theta, n, steps, iters, eval_bonus, fitness); break;

@@ -238,6 +238,27 @@ def test_group_tail_equals_static(dev, c, hidden, iters):
         assert ss.max().item() > 8  # members outlived the first chunk
 
 
+@pytest.mark.parametrize("c,hidden", [(1, 64), (2, 4), (2, 32)])
+def test_small_tail_bounds(dev, c, hidden):
+    """At C <= 2, populations and evaluations past 16 per CU run in 8-lane groups up to 32 per
+    CU, in 16-lane groups below and in chunks above: each bound, with ragged last waves, equals
+    the one-lane kernel and, for the evaluation, its slices."""
+    from hipenvs import legged, legged_rollout
+
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    theta = torch.from_numpy(_population(32 * cus + 2, c, hidden, 0.3, 9)).to(dev)
+    state = legged.Legged(c).reset(32 * cus + 2, seed=12, device=dev)
+    for p in (2, 16 * cus, 16 * cus + 2, 32 * cus, 32 * cus + 2):
+        s, th = state[:, :p].contiguous(), theta[:p]
+        got = legged_rollout.rollout(s, th, hidden, 40, c, schedule="chunked", chunk_steps=8, iters=4)
+        want = legged_rollout.rollout(s, th, hidden, 40, c, schedule="rows", iters=4)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), p
+        scores = legged_rollout.evaluate(s, theta[0], hidden, 60, c, 4)
+        slices = [legged_rollout.evaluate(s[:, i:i + 1000].contiguous(), theta[0], hidden, 60, c, 4)
+                  for i in range(0, p, 1000)]
+        assert torch.equal(scores, torch.cat(slices)), p
+
+
 @pytest.mark.parametrize("c,hidden,iters,above", [(1, 4, 8, 8), (2, 32, 8, 8), (3, 64, 8, 8), (4, 64, 8, 8),
                                                   (2, 64, 4, 8), (4, 64, 16, 8), (4, 4, 8, 8), (4, 32, 8, 8),
                                                   (4, 64, 8, 44), (2, 64, 8, 28)])
