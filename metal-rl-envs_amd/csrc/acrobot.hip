@@ -9,15 +9,12 @@
 // counter RNG of acrobot_metal.py:78-83. Per env-step the step kernel moves 41
 // algorithmic bytes; it is VALU-bound (14 sin/cos, 18 IEEE divisions).
 
+#include "acrobot_mass.h"
 #include "es_rollout.h"
 
 namespace hipenvs {
 namespace ac {
 
-constexpr float D1_C0 = 0x1p-2f;              // float32(1.0 * 0.5**2)
-constexpr float D1_C1 = 0x1.4p+0f;            // float32(1.0**2 + 0.5**2)
-constexpr float D2_C0 = 0x1p-2f;              // float32(0.5**2)
-constexpr float D2_C1 = 0x1p-1f;              // float32(1.0 * 0.5)
 constexpr float PHI2_C = 0x1.39999ap+2f;      // float32(1.0 * 0.5 * 9.8)
 constexpr float HALF_PI = 0x1.921fb6p+0f;     // float32(pi / 2)
 constexpr float PHI1_A = -0x1p-1f;            // float32(-1.0 * 1.0 * 0.5)
@@ -37,26 +34,24 @@ using S4 = roll::State4;  // theta1, theta2, dtheta1, dtheta2 (or their derivati
 
 // acrobot_np.py:64-84. The numpy expression's multiplications by the Python
 // float 1.0 (m2 *, 2 * l1 * lc2 *) are exact and omitted.
-// d1 lies in [2.5, 4.5] and d2 in [0.75, 1.75], so the two quotients of d2 are never subnormal
-// and divide through d1's float64 reciprocal directly (DivRecip's argument, with nothing to
-// mark). The other two divide with IEEE division: through a reciprocal, with a wave vote for
-// tiny numerators, the step gained nothing (6.37 against 6.22 us at N = 262,144) and the group
-// form lost (874 against 863 us a rollout). The three sin/cos share one range vote.
+// The two quotients of d2 by d1 come from d1's reciprocal estimate (acrobot_mass.h). The other two
+// divide with IEEE division: through a float64 reciprocal, with a wave vote for tiny numerators,
+// the step gained nothing (6.37 against 6.22 us at N = 262,144) and the group form lost (874
+// against 863 us a rollout). The three sin/cos share one range vote.
 __device__ __forceinline__ S4 dsdt(const S4& s, float torque) {
   const float ang[3] = {s.b, (s.a + s.b) - HALF_PI, s.a - HALF_PI};
   float sn[3], cs[3];
   det_sincos_small<3>(ang, sn, cs);
   const float s2 = sn[0], c2 = cs[0];
-  const float d1 = ((D1_C0 + (D1_C1 + c2)) + 1.0f) + 1.0f;
-  const double r1 = recip_normal(d1);
-  const float d2 = (D2_C0 + D2_C1 * c2) + 1.0f;
+  const float d1 = mass_d1(c2), d2 = mass_d2(c2);
+  const float r1 = __builtin_amdgcn_rcpf(d1);
   const float phi2 = PHI2_C * cs[1];
   const float t1 = (PHI1_A * (s.d * s.d)) * s2;
   const float t2 = (s.d * s.c) * s2;
   const float t3 = PHI1_C * cs[2];
   const float phi1 = ((t1 - t2) + t3) + phi2;
-  const float num = ((torque + (float)((double)d2 * r1) * phi1) - (DD2_C * (s.c * s.c)) * s2) - phi2;
-  const float den = DEN_C - (float)((double)(d2 * d2) * r1);
+  const float num = ((torque + mass_quotient(d2, d1, r1) * phi1) - (DD2_C * (s.c * s.c)) * s2) - phi2;
+  const float den = DEN_C - mass_quotient(d2 * d2, d1, r1);
   const float dd2 = num / den;
   const float dd1 = (-((d2 * dd2) + phi1)) / d1;
   return S4{s.c, s.d, dd1, dd2};
@@ -148,14 +143,13 @@ __device__ __forceinline__ S4 dsdt_group(const S4& s, float torque, int g) {
   float sn, cs;
   det_sincos(x, &sn, &cs);
   const float s2 = lane_bcast<G, 0>(sn), c2 = lane_bcast<G, 0>(cs);
-  const float d1 = ((D1_C0 + (D1_C1 + c2)) + 1.0f) + 1.0f;
-  const float d2 = (D2_C0 + D2_C1 * c2) + 1.0f;
+  const float d1 = mass_d1(c2), d2 = mass_d2(c2);
   const float phi2 = PHI2_C * lane_bcast<G, 1>(cs);
   const float t1 = (PHI1_A * (s.d * s.d)) * s2;
   const float t2 = (s.d * s.c) * s2;
   const float t3 = PHI1_C * lane_bcast<G, 2>(cs);
   const float phi1 = ((t1 - t2) + t3) + phi2;
-  const float q = ((g == 1) ? d2 * d2 : d2) / d1;  // lane 0: d2 / d1, lane 1: (d2 * d2) / d1
+  const float q = mass_quotient((g == 1) ? d2 * d2 : d2, d1, __builtin_amdgcn_rcpf(d1));  // lane 1: d2^2 / d1, else d2 / d1
   const float num = ((torque + lane_bcast<G, 0>(q) * phi1) - (DD2_C * (s.c * s.c)) * s2) - phi2;
   const float den = DEN_C - lane_bcast<G, 1>(q);
   const float dd2 = num / den;

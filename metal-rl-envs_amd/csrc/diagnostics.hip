@@ -3,7 +3,7 @@
 // the device bit for bit (deterministic sin/cos/tanh; division through a float64
 // reciprocal with its subnormal redo).
 
-#include "hipenvs_device.h"
+#include "acrobot_mass.h"
 
 namespace hipenvs {
 namespace diag {
@@ -88,7 +88,8 @@ __device__ __forceinline__ bool same_bits(float a, float b) {
 // Every float32 bit pattern first + i, i < count: counts[0] det_tanh against its plain form,
 // counts[1] the float32 argument reduction against its plain form (|x| <= 256), counts[2]
 // sqrt_pivot's root against IEEE sqrtf (positive normals), counts[3] its reciprocal and
-// recip_normal's against 1 / x in float64, beyond 2^-51 relative (positive normals below 2^126).
+// recip_normal's against 1 / x in float64, beyond 2^-51 relative (positive normals below 2^126),
+// and Acrobot's quotients at cos(theta2) = x against IEEE division (|x| <= 1.5).
 __global__ __launch_bounds__(kBlock) void arith_check_kernel(uint64_t first, uint64_t count,
                                                              unsigned long long* __restrict__ counts) {
   const uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
@@ -107,6 +108,11 @@ __global__ __launch_bounds__(kBlock) void arith_check_kernel(uint64_t first, uin
     const double e_root = fabs(__builtin_fma(-(double)y, r, 1.0));
     const double e_recip = fabs(__builtin_fma(-(double)x, recip_normal(x), 1.0));
     if (!(e_root <= 0x1p-51) || !(e_recip <= 0x1p-51)) atomicAdd(&counts[3], 1ull);
+  }
+  if (fabsf(x) <= 1.5f) {
+    const float d1 = ac::mass_d1(x), d2 = ac::mass_d2(x), r = __builtin_amdgcn_rcpf(d1);
+    if (!same_bits(ac::mass_quotient(d2, d1, r), d2 / d1) || !same_bits(ac::mass_quotient(d2 * d2, d1, r), (d2 * d2) / d1))
+      atomicAdd(&counts[3], 1ull);
   }
 }
 
