@@ -349,11 +349,11 @@ def module_api_rate(n, steps, dev):
 # headline loop, the step alone and the bounded sweep's graphs), in ns;
 # profiles/cartpole_step_n262144.md tabulates them. The tracer runs each dispatch on its own,
 # so these include the per-dispatch ramp and drain that back-to-back launches overlap.
-CARTPOLE_TRACE_NS = {1 << 18: 3330.8, 1 << 20: 8376.5, 1 << 24: 111245.2}
+CARTPOLE_TRACE_NS = {1 << 18: 3324.4, 1 << 20: 8365.1, 1 << 24: 110643.4}
 # sha256 (first 16 hex digits) of the sources the traced kernel was built from,
 # csrc/cartpole.hip then csrc/hipenvs_device.h: when the sources differ, the trace no longer
 # describes this build, and cartpole_roofline falls back to the run's own HIP-event figure.
-CARTPOLE_TRACE_SOURCE_SHA = "0a1e787657580dc3"
+CARTPOLE_TRACE_SOURCE_SHA = "cd99110bc14ef4e1"
 CARTPOLE_TRACE_SOURCES = ("metal-rl-envs_amd/csrc/cartpole.hip", "metal-rl-envs_amd/csrc/hipenvs_device.h")
 
 
