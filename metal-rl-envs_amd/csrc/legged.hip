@@ -528,17 +528,19 @@ __host__ __device__ constexpr int64_t round_to_tile(int64_t n) { return (n + kTi
 // step, which is what bounds the tail. Results are those of the one-lane schedule, bit for bit.
 // At C <= 2 every lane role also fits in 8 lanes (2C + 1 solves, C^2 Delassus blocks, 3C
 // heads), eight members to a wave. A step is longer that way (two moves a broadcast, twice the
-// hidden units a lane), but one launch holds twice the members: it runs populations of 16 to 32
-// members per CU, which then need no chunks. H = 32, 300 steps, 8 sweeps, ms (8 lanes / 16):
-//   biped, P = 4,096 standing 3.50 / 3.06, falling 3.42 / 3.08; P = 8,192 standing 3.51 / 4.36,
-//   falling 3.49 / 3.23; P = 65,536 falling 4.54 / 4.20; H = 64, P = 262,144 7.10 / 6.67
-//   one leg, P = 4,096 0.65 / 0.58; P = 262,144 3.66 / 3.60
+// hidden units a lane), but one launch holds twice the members, so populations past 16 members
+// per CU take it from 32 survivors per CU on. H = 32, 300 steps, 8 sweeps, ms (8 lanes / 16 with
+// 4-lane chunks above 16 per CU): biped, P = 4,096 standing 3.50 / 3.06, falling 3.42 / 3.08;
+// P = 8,192 standing 3.51 / 4.36; one leg, P = 4,096 0.65 / 0.58. At P = 262,144, H = 64, 1,000
+// steps, where 16 to 32 bipeds per CU last for most of the horizon, 16 sweeps take
+// 26.1 / 28.7 ms and 4 sweeps 16.4 / 17.4; 8-lane chunks between, without resident weights,
+// 29.6 and 17.5.
 constexpr int kTailLanes = 16, kSmallTailLanes = 8;
 constexpr int64_t kTailPerCu = 4 * (64 / kTailLanes), kSmallTailPerCu = 4 * (64 / kSmallTailLanes);
-// Whether n members or envs on `cus` CUs take the 8-lane form.
+// Whether the tail of a population of p takes the 8-lane form.
 template <int C>
-inline bool small_tail(int64_t n, int cus) {
-  return C <= 2 && n > kTailPerCu * cus && n <= kSmallTailPerCu * cus;
+inline bool small_tail(int64_t p, int cus) {
+  return C <= 2 && p > kTailPerCu * cus;
 }
 // Above the tail's bound and up to this many survivors per CU, a chunk runs in the group form
 // (rollout_group_chunk_kernel) instead of one member per lane, with LEGGED_GROUP_CHUNK_LANES
@@ -1360,7 +1362,7 @@ int launch_evaluate(int32_t hidden, const float* state, const float* theta, int6
     if (n <= kTailPerCu * cus)
       return launch_evaluate_group<C, kTailLanes>(hidden, state, theta, n, steps, iters, eval_bonus, fitness, s);
     if constexpr (C <= 2) {
-      if (small_tail<C>(n, cus))
+      if (n <= kSmallTailPerCu * cus)
         return launch_evaluate_group<C, kSmallTailLanes>(hidden, state, theta, n, steps, iters, eval_bonus, fitness, s);
     }
   }
