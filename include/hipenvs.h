@@ -393,8 +393,8 @@ int hipenvs_sqrt_recip_check(uint64_t first, uint64_t count, unsigned long long*
  * kernels' shortened arithmetic: adds to counts[0] the inputs whose tanh differs from the
  * same polynomial with every product rounded and IEEE division, to counts[1] those (|x| <=
  * 256) whose sin/cos argument reduction differs from the unfused one, to counts[2] the
- * positive normals whose Cholesky pivot root differs from IEEE sqrtf, and to counts[3] those
- * (below 2^126) whose float64 pivot or divisor reciprocal is off by more than 2^-51 and the
+ * positive finite ones whose Cholesky pivot root differs from IEEE sqrtf, and to counts[3] those
+ * whose float64 pivot or divisor reciprocal is off by more than 2^-51 and the
  * cosines of theta2 (|x| <= 1.5) at which Acrobot's quotients of its mass matrix differ from
  * IEEE division. counts: four values of device memory the caller zeroes. */
 int hipenvs_arith_check(uint64_t first, uint64_t count, unsigned long long* counts,

@@ -87,8 +87,8 @@ __device__ __forceinline__ bool same_bits(float a, float b) {
 
 // Every float32 bit pattern first + i, i < count: counts[0] det_tanh against its plain form,
 // counts[1] the float32 argument reduction against its plain form (|x| <= 256), counts[2]
-// sqrt_pivot's root against IEEE sqrtf (positive normals), counts[3] its reciprocal and
-// recip_normal's against 1 / x in float64, beyond 2^-51 relative (positive normals below 2^126),
+// sqrt_pivot's root against IEEE sqrtf (positive and finite x), counts[3] its reciprocal and
+// recip_normal's against 1 / x in float64, beyond 2^-51 relative (the same x),
 // and Acrobot's quotients at cos(theta2) = x against IEEE division (|x| <= 1.5).
 __global__ __launch_bounds__(kBlock) void arith_check_kernel(uint64_t first, uint64_t count,
                                                              unsigned long long* __restrict__ counts) {
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(kBlock) void arith_check_kernel(uint64_t first, uin
     const float ra = reduce_small(x, &qa), rb = reduce_plain(x, &qb);
     if (!same_bits(ra, rb) || qa != qb) atomicAdd(&counts[1], 1ull);
   }
-  if (x >= 0x1p-126f && x < 0x1p+126f) {
+  if (x > 0.0f && x < __builtin_inff()) {
     double r;
     const float y = sqrt_pivot(x, &r);
     if (!same_bits(y, sqrtf(x))) atomicAdd(&counts[2], 1ull);

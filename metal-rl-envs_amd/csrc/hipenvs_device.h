@@ -403,12 +403,13 @@ __device__ __forceinline__ float sqrt_rn(float x) {
   return __builtin_amdgcn_classf(x, 0x260) ? x : y;  // class bits 5, 6, 9: -0, +0, +inf
 }
 
-// Float64 reciprocal of a float32 d that is normal and finite (or NaN, which stays NaN) for
+// Float64 reciprocal of a float32 d that is finite and not 0 (or NaN, which stays NaN) for
 // DivRecip: the hardware estimate r0 and one third-order step,
 // r0 + r0 (e + e^2) with e = 1 - d r0 (|e| < 2^-20, so the truncation is below 2^-60 and the
 // result is within an ulp of 1 / d). Five instructions where recip() takes nine: a quotient
-// needs the reciprocal only to well within 2^-50 (see above), not correctly rounded, and these
-// divisors are never 0 or infinite.
+// needs the reciprocal only to well within 2^-50 (see above), not correctly rounded. For
+// d = +-0 or +-inf it is NaN where recip() is +-inf or +-0: for divisors that cannot be, or
+// whose quotients by them come out NaN either way.
 __device__ __forceinline__ double recip_normal(float d) {
   const double x = (double)d;
   const double r0 = __builtin_amdgcn_rcp(x);
@@ -417,12 +418,16 @@ __device__ __forceinline__ double recip_normal(float d) {
 }
 
 // The square root y = sqrtf(s) of a Cholesky pivot and the float64 reciprocal of y, for s
-// normal, finite and positive (or NaN). The mass matrices here depend on the angles alone
-// through their sines and cosines and are positive definite over that compact set, the smallest
-// pivot 0.0625 (legged) and 0.5 (pendulum), so s is never 0 or infinite. y is sqrt_rn without its
-// special cases; its reciprocal starts from the same estimate r of 1 / sqrt(s) (y differs
-// from sqrt(s) by half an ulp, so 1 - y r is below 2^-20) and takes one third-order step. Eleven
-// instructions and one transcendental where sqrt_rn and recip take eighteen and two.
+// positive and finite (or negative or NaN, both NaN then): sqrt_rn without its special cases;
+// the reciprocal starts from the same estimate r of 1 / sqrt(s) (y differs from sqrt(s) by half
+// an ulp, so 1 - y r is below 2^-20) and takes one third-order step. Eleven instructions and
+// one transcendental where sqrt_rn and recip take eighteen and two. The mass matrices here
+// depend on the angles alone through their sines and cosines, with pivots of at least 0.0625
+// (legged) and 0.5 (pendulum) while those are; but past about 2^50 det_sincos's reduction is no
+// longer within pi/4, its polynomials leave [-1, 1] with it, and a pivot can round to 0 or
+// overflow. sqrt_pivot gives NaN there, and with it every component of a solve up to that
+// pivot's own, where sqrt_rn goes on with 0 or infinity; so the callers take a NaN from finite
+// angles for a pivot of that kind and evaluate again with DivIEEE.
 __device__ __forceinline__ float sqrt_pivot(float s, double* recip_out) {
   const double d = (double)s;
   const double r = __builtin_amdgcn_rsq(d);
@@ -434,6 +439,8 @@ __device__ __forceinline__ float sqrt_pivot(float s, double* recip_out) {
   return y;
 }
 
+// How a body divides by a shared divisor and takes a pivot's root: through float64 reciprocals
+// (DivRecip), or IEEE throughout (DivIEEE).
 struct DivRecip {
   static constexpr bool kRecip = true;  // divides by multiplying with r; d is not read
   // Per lane, the least (bits << 1) - 2 over the quotients, in uint32 arithmetic: the shift
@@ -447,12 +454,17 @@ struct DivRecip {
     least = key < least ? key : least;
     return q;
   }
+  __device__ __forceinline__ float root(float s, double* recip_out) { return sqrt_pivot(s, recip_out); }
   __device__ __forceinline__ bool saw_subnormal() const { return least <= 0x00FFFFFCu; }
 };
 
 struct DivIEEE {
   static constexpr bool kRecip = false;
   __device__ __forceinline__ float operator()(float a, float d, double /*r*/) const { return a / d; }
+  __device__ __forceinline__ float root(float s, double* recip_out) const {
+    *recip_out = 0.0;  // not read
+    return sqrt_rn(s);
+  }
 };
 
 // Per-step streams (an action or torque row read once, reward and done rows written once)

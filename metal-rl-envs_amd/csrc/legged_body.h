@@ -277,7 +277,7 @@ __device__ __forceinline__ void substep(float (&q)[3 + C], float (&v)[3 + C], co
 #pragma unroll
       for (int p = 0; p < j; ++p) s = s - L[i][p] * L[j][p];
       if (i == j) {
-        L[i][i] = sqrt_pivot(s, &rL[i]);
+        L[i][i] = div.root(s, &rL[i]);
       } else {
         L[i][j] = div(s, L[j][j], rL[j]);
       }
@@ -667,9 +667,21 @@ __device__ __forceinline__ void substep(float (&q)[3 + C], float (&v)[3 + C], co
   }
 }
 
+// Whether every foot's angle is finite, so that a mass matrix entry that is not comes from
+// det_sincos's range (sqrt_pivot) and not from a NaN or an infinity in the state.
+template <int C>
+__device__ __forceinline__ bool finite_angles(const float (&q)[3 + C]) {
+  bool ok = true;
+#pragma unroll
+  for (int k = 0; k < C; ++k) ok &= fabsf(q[2] + q[3 + k]) < __builtin_inff();
+  return ok;
+}
+
 // One substep dividing through the shared float64 reciprocals; a lane on which a quotient
-// came out subnormal (never met in practice) redoes the substep from its saved state with
-// IEEE division, so the result is always the IEEE one.
+// came out subnormal, or a pivot was 0 or infinite (neither met in practice), redoes the
+// substep from its saved state with IEEE division and roots, so the result is always the IEEE
+// one. Such a pivot leaves NaN in every velocity from finite angles; once the state itself is
+// NaN both forms are.
 template <int C, bool kHopperSum = false, bool kStage = false>
 __device__ __forceinline__ void substep_exact(float (&q)[3 + C], float (&v)[3 + C], const float (&tq)[C], int iters,
                                               float assist, float assist_damping, float* stage = nullptr) {
@@ -682,7 +694,7 @@ __device__ __forceinline__ void substep_exact(float (&q)[3 + C], float (&v)[3 + 
   }
   DivRecip fast;
   substep<C, DivRecip, 0, kHopperSum, kStage>(q, v, tq, iters, assist, assist_damping, fast, stage);
-  if (fast.saw_subnormal()) {
+  if (fast.saw_subnormal() || (v[2] != v[2] && finite_angles<C>(q0))) {
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       q[i] = q0[i];
@@ -693,9 +705,9 @@ __device__ __forceinline__ void substep_exact(float (&q)[3 + C], float (&v)[3 + 
   }
 }
 
-// The group form of substep_exact: the fast divisions, and when any live lane of the wave saw
-// a subnormal quotient the whole wave redoes the substep with IEEE division (identical bits
-// wherever nothing was marked), which keeps the group's barriers in uniform control flow.
+// The group form of substep_exact: the fast form, and when any live lane of the wave has to
+// redo the substep the whole wave does (identical bits wherever nothing called for it), which
+// keeps the group's barriers in uniform control flow.
 template <int C, int G>
 __device__ __forceinline__ void substep_exact_group(float (&q)[3 + C], float (&v)[3 + C], const float (&tq)[C],
                                                     int iters, float assist, float assist_damping, float* xs, int g,
@@ -709,7 +721,9 @@ __device__ __forceinline__ void substep_exact_group(float (&q)[3 + C], float (&v
   }
   DivRecip fast;
   substep<C, DivRecip, G>(q, v, tq, iters, assist, assist_damping, fast, xs, g, xd);
-  if (__any(live && fast.saw_subnormal())) {  // lanes of finished members step on, unused
+  const bool nan = v[2] != v[2];
+  if (__any(live && (fast.saw_subnormal() || nan)) &&  // lanes of finished members step on, unused
+      __any(live && (fast.saw_subnormal() || (nan && finite_angles<C>(q0))))) {
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       q[i] = q0[i];

@@ -214,7 +214,7 @@ __device__ __forceinline__ void mass_matrix_accelerations_with(const float* th, 
 #pragma unroll
       for (int p = 0; p < j; ++p) t = t - L[i][p] * L[j][p];
       if (i == j) {
-        L[i][i] = sqrt_pivot(t, &rL[i]);
+        L[i][i] = div.root(t, &rL[i]);
       } else {
         L[i][j] = div(t, L[j][j], rL[j]);
       }
@@ -238,7 +238,8 @@ __device__ __forceinline__ void mass_matrix_accelerations_with(const float* th, 
 
 // The mass-matrix model's accelerations (pendulum_np.py:69-95). Divisions go through the
 // pivots' shared float64 reciprocals (DivRecip: the IEEE quotient unless it is subnormal);
-// a lane on which a quotient came out subnormal evaluates again with IEEE division. RK4 at
+// a lane on which a quotient came out subnormal, or a pivot was 0 or infinite (NaN from finite
+// angles, sqrt_pivot), evaluates again with IEEE division and roots. RK4 at
 // N = 65,536: K = 16 55.5 -> 48.4 us per step, K = 8 16.1 -> 15.2, K = 4 6.85 -> 6.63; at
 // K = 2 (3.97 -> 4.17 us) it divides with IEEE division alone.
 template <int K>
@@ -247,7 +248,14 @@ __device__ __forceinline__ void mass_matrix_accelerations(const float* th, const
   if constexpr (K > 2) {
     DivRecip fast;
     mass_matrix_accelerations_with<K>(th, om, torque, acc, fast);
-    if (fast.saw_subnormal()) {
+    bool redo = fast.saw_subnormal();
+    if (acc[0] != acc[0]) {
+      bool finite = true;
+#pragma unroll
+      for (int i = 0; i < K; ++i) finite &= fabsf(th[i]) < __builtin_inff();
+      redo |= finite;
+    }
+    if (redo) {
       DivIEEE ieee;
       mass_matrix_accelerations_with<K>(th, om, torque, acc, ieee);
     }

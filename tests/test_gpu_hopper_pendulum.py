@@ -98,6 +98,25 @@ def test_pendulum_step_matches_oracle(dev, k):
     np.testing.assert_array_equal(to_np(nxt), e_next)
 
 
+@pytest.mark.parametrize("k", [1, 2, 4, 16])
+def test_pendulum_accelerations_past_the_sincos_reduction(dev, k):
+    """One angle of 1e17 to 1e20: det_sincos's reduction has no digits left there, its
+    polynomials leave [-1, 1], and a pivot of the mass matrix can round to 0 (in 1 to 2 % of
+    these states), which the oracle's square root and divisions carry on."""
+    from hipenvs import pendulum
+
+    n = 4000
+    state, _ = pendulum_states(k, n, seed=k)
+    r = np.random.default_rng(k)
+    state[r.integers(0, k, n), np.arange(n)] = (10.0 ** r.uniform(17, 20, n)).astype(np.float32)
+    with np.errstate(all="ignore"):
+        want = op.mass_matrix_dsdt(state, np.ones(n, np.float32), k, trig="det")[k:]
+    got = pendulum.Pendulum(k).accelerations(torch.from_numpy(state).to(dev), torch.ones(n, device=dev))
+    finite = np.isfinite(want).all(0)
+    assert finite.sum() > n // 10
+    np.testing.assert_array_equal(to_np(got)[:, finite], want[:, finite])
+
+
 def test_pendulum_step_at_the_benchmark_size(dev):
     """K = 16 at N = 65,536, the bench's largest mass-matrix pendulum shape."""
     from hipenvs import pendulum

@@ -95,6 +95,35 @@ def test_step_forms_give_the_same_bits(dev, c, iters, assist):
                                           np.signbit(want[..., :m][zeros].astype(np.float32)))
 
 
+@pytest.mark.parametrize("c", [1, 2, 4])
+def test_step_with_angles_past_the_sincos_reduction(dev, c):
+    """Torso angles of 1e17 to 1e20: det_sincos's reduction has no digits left there and its
+    polynomials leave [-1, 1], so a mass-matrix pivot can round to 0 (in about 1 % of these
+    envs for C >= 2), which the oracle's square root and divisions carry on. Every lane-group
+    form of the step equals the oracle wherever the oracle's step is finite (elsewhere the
+    kernels leave out products with an exact 0)."""
+    from hipenvs import legged
+
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    n = 64 * cus + 1
+    state, action = legged_states(c, n, seed=60 + c)
+    r = np.random.default_rng(70 + c)
+    state[2] = (10.0 ** r.uniform(17, 20, n) * r.choice([-1, 1], n)).astype(np.float32)
+    state[5 + c:] = 0
+    oracle = olg.Legged(c, 2)
+    with np.errstate(all="ignore"):
+        finite = np.isfinite(oracle.physics(state, action)).all(0)
+        want = oracle.step(state, action, seed=4)
+    assert finite.sum() > n // 10
+    dstate, daction = torch.from_numpy(state).to(dev), torch.from_numpy(action.astype(np.int32)).to(dev)
+    body = legged.Legged(c, 2)
+    for m in (n, 64 * cus, 16 * cus):
+        body.reseed(3)
+        got = body.step(dstate[:, :m].contiguous(), daction[:m])
+        for g, w in zip(got, want):
+            np.testing.assert_array_equal(to_np(g)[..., finite[:m]], w[..., :m][..., finite[:m]])
+
+
 @pytest.mark.parametrize("c", [2, 4])
 def test_step_with_assist_matches_oracle(dev, c):
     from hipenvs import legged
