@@ -7,7 +7,8 @@
 // (each constant's defining expression is beside it); RK4/wrap/clip follow
 // acrobot_np.py:47-61,87-89, termination acrobot_np.py:92-93, reset the
 // counter RNG of acrobot_metal.py:78-83. Per env-step the step kernel moves 41
-// algorithmic bytes; it is VALU-bound (14 sin/cos, 18 IEEE divisions).
+// algorithmic bytes; it is VALU-bound (14 sin/cos, 18 divisions, of which 8
+// through a reciprocal estimate).
 
 #include "acrobot_mass.h"
 #include "es_rollout.h"
@@ -34,15 +35,23 @@ using S4 = roll::State4;  // theta1, theta2, dtheta1, dtheta2 (or their derivati
 
 // acrobot_np.py:64-84. The numpy expression's multiplications by the Python
 // float 1.0 (m2 *, 2 * l1 * lc2 *) are exact and omitted.
-// The two quotients of d2 by d1 come from d1's reciprocal estimate (acrobot_mass.h). The other two
+// The two quotients of d2 by d1 come from d1's reciprocal estimate (acrobot_mass.h), or with
+// kInRange false from IEEE division; `reach` keeps the largest |cos(theta2)| met. The other two
 // divide with IEEE division: through a float64 reciprocal, with a wave vote for tiny numerators,
 // the step gained nothing (6.37 against 6.22 us at N = 262,144) and the group form lost (874
 // against 863 us a rollout). The three sin/cos share one range vote.
-__device__ __forceinline__ S4 dsdt(const S4& s, float torque) {
+template <bool kInRange>
+__device__ __forceinline__ S4 dsdt(const S4& s, float torque, float& reach) {
   const float ang[3] = {s.b, (s.a + s.b) - HALF_PI, s.a - HALF_PI};
   float sn[3], cs[3];
-  det_sincos_small<3>(ang, sn, cs);
+  if constexpr (kInRange) {
+    det_sincos_small<3>(ang, sn, cs);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) det_sincos(ang[i], &sn[i], &cs[i]);
+  }
   const float s2 = sn[0], c2 = cs[0];
+  reach = fmaxf(reach, fabsf(c2));
   const float d1 = mass_d1(c2), d2 = mass_d2(c2);
   const float r1 = __builtin_amdgcn_rcpf(d1);
   const float phi2 = PHI2_C * cs[1];
@@ -50,8 +59,8 @@ __device__ __forceinline__ S4 dsdt(const S4& s, float torque) {
   const float t2 = (s.d * s.c) * s2;
   const float t3 = PHI1_C * cs[2];
   const float phi1 = ((t1 - t2) + t3) + phi2;
-  const float num = ((torque + mass_quotient(d2, d1, r1) * phi1) - (DD2_C * (s.c * s.c)) * s2) - phi2;
-  const float den = DEN_C - mass_quotient(d2 * d2, d1, r1);
+  const float num = ((torque + mass_quotient<kInRange>(d2, d1, r1) * phi1) - (DD2_C * (s.c * s.c)) * s2) - phi2;
+  const float den = DEN_C - mass_quotient<kInRange>(d2 * d2, d1, r1);
   const float dd2 = num / den;
   const float dd1 = (-((d2 * dd2) + phi1)) / d1;
   return S4{s.c, s.d, dd1, dd2};
@@ -61,20 +70,97 @@ constexpr double INV_TWO_PI = 1.0 / (double)TWO_PI;  // for div_const(x, .) == x
 
 __device__ __forceinline__ float wrap(float x) { return x - TWO_PI * floorf(div_const(x + PI, INV_TWO_PI)); }
 
-// RK4 + wrap + clip in place (acrobot_np.py:47-61).
-__device__ __forceinline__ void rk4(S4& s, float torque) {
-  const S4 k1 = dsdt(s, torque);
-  const S4 k2 = dsdt(S4{s.a + DT_2 * k1.a, s.b + DT_2 * k1.b, s.c + DT_2 * k1.c, s.d + DT_2 * k1.d}, torque);
-  const S4 k3 = dsdt(S4{s.a + DT_2 * k2.a, s.b + DT_2 * k2.b, s.c + DT_2 * k2.c, s.d + DT_2 * k2.d}, torque);
-  const S4 k4 = dsdt(S4{s.a + DT * k3.a, s.b + DT * k3.b, s.c + DT * k3.c, s.d + DT * k3.d}, torque);
-  const float na = s.a + DT_6 * (((k1.a + 2.0f * k2.a) + 2.0f * k3.a) + k4.a);
-  const float nb = s.b + DT_6 * (((k1.b + 2.0f * k2.b) + 2.0f * k3.b) + k4.b);
-  const float nc = s.c + DT_6 * (((k1.c + 2.0f * k2.c) + 2.0f * k3.c) + k4.c);
-  const float nd = s.d + DT_6 * (((k1.d + 2.0f * k2.d) + 2.0f * k3.d) + k4.d);
-  s.a = wrap(na);
-  s.b = wrap(nb);
-  s.c = clip(nc, -MAX_VEL_1, MAX_VEL_1);
-  s.d = clip(nd, -MAX_VEL_2, MAX_VEL_2);
+// The group's physics, with the transcendentals and the two quotients by d1 spread over the
+// group's lanes: lanes 0, 1, 2 evaluate one det_sincos each (one instruction stream for the
+// three) and every lane of the 16-lane group (one DPP row) receives the results by row
+// broadcast. Each value is the single-lane function's on the same argument, so the bits
+// are those of dsdt/rk4/terminal.
+struct GroupTrig {
+  float sin_a, cos_a, sin_b, cos_b, cos_ab;  // theta1, theta2, theta2 + theta1
+};
+
+template <int G>
+__device__ __forceinline__ GroupTrig group_trig(const S4& s, int g) {
+  const float x = (g == 1) ? s.b : (g == 2) ? (s.b + s.a) : s.a;
+  float sn, cs;
+  det_sincos(x, &sn, &cs);
+  return GroupTrig{lane_bcast<G, 0>(sn), lane_bcast<G, 0>(cs), lane_bcast<G, 1>(sn), lane_bcast<G, 1>(cs),
+                   lane_bcast<G, 2>(cs)};
+}
+
+template <int G, bool kInRange>
+__device__ __forceinline__ S4 dsdt_group(const S4& s, float torque, int g, float& reach) {
+  const float x = (g == 1) ? ((s.a + s.b) - HALF_PI) : (g == 2) ? (s.a - HALF_PI) : s.b;
+  float sn, cs;
+  det_sincos(x, &sn, &cs);
+  const float s2 = lane_bcast<G, 0>(sn), c2 = lane_bcast<G, 0>(cs);
+  reach = fmaxf(reach, fabsf(c2));
+  const float d1 = mass_d1(c2), d2 = mass_d2(c2);
+  const float phi2 = PHI2_C * lane_bcast<G, 1>(cs);
+  const float t1 = (PHI1_A * (s.d * s.d)) * s2;
+  const float t2 = (s.d * s.c) * s2;
+  const float t3 = PHI1_C * lane_bcast<G, 2>(cs);
+  const float phi1 = ((t1 - t2) + t3) + phi2;
+  // lane 1: d2^2 / d1, else d2 / d1
+  const float q = mass_quotient<kInRange>((g == 1) ? d2 * d2 : d2, d1, __builtin_amdgcn_rcpf(d1));
+  const float num = ((torque + lane_bcast<G, 0>(q) * phi1) - (DD2_C * (s.c * s.c)) * s2) - phi2;
+  const float den = DEN_C - lane_bcast<G, 1>(q);
+  const float dd2 = num / den;
+  const float dd1 = (-((d2 * dd2) + phi1)) / d1;
+  return S4{s.c, s.d, dd1, dd2};
+}
+
+template <int G, bool kInRange>
+__device__ __forceinline__ S4 derivative(const S4& s, float torque, int g, float& reach) {
+  if constexpr (G == 1)
+    return dsdt<kInRange>(s, torque, reach);
+  else
+    return dsdt_group<G, kInRange>(s, torque, g, reach);
+}
+
+// RK4 (acrobot_np.py:47-61) from s, before the wrap and clip. The out-of-range form, which no
+// ordinary state takes, is a rolled loop, so that it costs the other neither registers nor the
+// instruction cache (unrolled it took 10 registers more: one lane at H = 8 fell from four waves per
+// SIMD to three; a choice in each derivative instead, under the sin/cos vote, took the 16-lane
+// rollout at P = 4,096 from 806 to 931 us).
+template <int G, bool kInRange>
+__device__ __forceinline__ S4 rk4_unwrapped(const S4& s, float torque, int g, float& reach) {
+  S4 sum{}, x = s;
+  if constexpr (kInRange) {
+    const S4 k1 = derivative<G, true>(s, torque, g, reach);
+    const S4 k2 = derivative<G, true>(
+        S4{s.a + DT_2 * k1.a, s.b + DT_2 * k1.b, s.c + DT_2 * k1.c, s.d + DT_2 * k1.d}, torque, g, reach);
+    const S4 k3 = derivative<G, true>(
+        S4{s.a + DT_2 * k2.a, s.b + DT_2 * k2.b, s.c + DT_2 * k2.c, s.d + DT_2 * k2.d}, torque, g, reach);
+    const S4 k4 = derivative<G, true>(
+        S4{s.a + DT * k3.a, s.b + DT * k3.b, s.c + DT * k3.c, s.d + DT * k3.d}, torque, g, reach);
+    sum = S4{((k1.a + 2.0f * k2.a) + 2.0f * k3.a) + k4.a, ((k1.b + 2.0f * k2.b) + 2.0f * k3.b) + k4.b,
+             ((k1.c + 2.0f * k2.c) + 2.0f * k3.c) + k4.c, ((k1.d + 2.0f * k2.d) + 2.0f * k3.d) + k4.d};
+  } else {
+#pragma unroll 1
+    for (int i = 0; i < 4; ++i) {
+      const S4 k = derivative<G, false>(x, torque, g, reach);
+      const float w = (i == 1 || i == 2) ? 2.0f : 1.0f, h = (i == 2) ? DT : DT_2;
+      sum = S4{i ? sum.a + w * k.a : k.a, i ? sum.b + w * k.b : k.b, i ? sum.c + w * k.c : k.c,
+               i ? sum.d + w * k.d : k.d};
+      x = S4{s.a + h * k.a, s.b + h * k.b, s.c + h * k.c, s.d + h * k.d};
+    }
+  }
+  return S4{s.a + DT_6 * sum.a, s.b + DT_6 * sum.b, s.c + DT_6 * sum.c, s.d + DT_6 * sum.d};
+}
+
+// RK4 + wrap + clip in place (acrobot_np.py:47-61) on G lanes. When a cosine on any lane left the
+// range that the short quotients are exact over (angles past about 2^50, see acrobot_mass.h), the
+// wave evaluates again with IEEE division: the same bits for the others.
+template <int G>
+__device__ __forceinline__ void rk4(S4& s, float torque, int g = 0) {
+  float reach = 0.0f;
+  S4 x = rk4_unwrapped<G, true>(s, torque, g, reach);
+  if (__builtin_expect(!wave_all(!(reach > kMassRange)), 0)) x = rk4_unwrapped<G, false>(s, torque, g, reach);
+  s.a = wrap(x.a);
+  s.b = wrap(x.b);
+  s.c = clip(x.c, -MAX_VEL_1, MAX_VEL_1);
+  s.d = clip(x.d, -MAX_VEL_2, MAX_VEL_2);
 }
 
 // acrobot_np.py:92-93: -cos(th1) - cos(th2 + th1) > 1.
@@ -102,7 +188,7 @@ __global__ __launch_bounds__(kBlock) void step_kernel(const float* __restrict__ 
   if (i >= n) return;
   S4 s{state[i], state[n + i], state[2 * n + i], state[3 * n + i]};
   const float torque = (float)(stream_load(action + i) - 1);
-  rk4(s, torque);
+  rk4<1>(s, torque);
   const bool d = terminal(s);
   if (d) {  // fresh draws only on terminated lanes; the reference selects (acrobot_metal.py:76-80)
     const uint32_t h = env_hash(seed, (uint32_t)i);
@@ -117,60 +203,6 @@ __global__ __launch_bounds__(kBlock) void step_kernel(const float* __restrict__ 
   next[3 * n + i] = s.d;
   stream_store(d ? 0.0f : -1.0f, reward + i);
   stream_store((uint8_t)(d ? 1 : 0), done + i);
-}
-
-// The group's physics, with the transcendentals and the two quotients by d1 spread over the
-// group's lanes: lanes 0, 1, 2 evaluate one det_sincos each (one instruction stream for the
-// three) and every lane of the 16-lane group (one DPP row) receives the results by row
-// broadcast. Each value is the single-lane function's on the same argument, so the bits
-// are those of dsdt/rk4/terminal.
-struct GroupTrig {
-  float sin_a, cos_a, sin_b, cos_b, cos_ab;  // theta1, theta2, theta2 + theta1
-};
-
-template <int G>
-__device__ __forceinline__ GroupTrig group_trig(const S4& s, int g) {
-  const float x = (g == 1) ? s.b : (g == 2) ? (s.b + s.a) : s.a;
-  float sn, cs;
-  det_sincos(x, &sn, &cs);
-  return GroupTrig{lane_bcast<G, 0>(sn), lane_bcast<G, 0>(cs), lane_bcast<G, 1>(sn), lane_bcast<G, 1>(cs),
-                   lane_bcast<G, 2>(cs)};
-}
-
-template <int G>
-__device__ __forceinline__ S4 dsdt_group(const S4& s, float torque, int g) {
-  const float x = (g == 1) ? ((s.a + s.b) - HALF_PI) : (g == 2) ? (s.a - HALF_PI) : s.b;
-  float sn, cs;
-  det_sincos(x, &sn, &cs);
-  const float s2 = lane_bcast<G, 0>(sn), c2 = lane_bcast<G, 0>(cs);
-  const float d1 = mass_d1(c2), d2 = mass_d2(c2);
-  const float phi2 = PHI2_C * lane_bcast<G, 1>(cs);
-  const float t1 = (PHI1_A * (s.d * s.d)) * s2;
-  const float t2 = (s.d * s.c) * s2;
-  const float t3 = PHI1_C * lane_bcast<G, 2>(cs);
-  const float phi1 = ((t1 - t2) + t3) + phi2;
-  const float q = mass_quotient((g == 1) ? d2 * d2 : d2, d1, __builtin_amdgcn_rcpf(d1));  // lane 1: d2^2 / d1, else d2 / d1
-  const float num = ((torque + lane_bcast<G, 0>(q) * phi1) - (DD2_C * (s.c * s.c)) * s2) - phi2;
-  const float den = DEN_C - lane_bcast<G, 1>(q);
-  const float dd2 = num / den;
-  const float dd1 = (-((d2 * dd2) + phi1)) / d1;
-  return S4{s.c, s.d, dd1, dd2};
-}
-
-template <int G>
-__device__ __forceinline__ void rk4_group(S4& s, float torque, int g) {
-  const S4 k1 = dsdt_group<G>(s, torque, g);
-  const S4 k2 = dsdt_group<G>(S4{s.a + DT_2 * k1.a, s.b + DT_2 * k1.b, s.c + DT_2 * k1.c, s.d + DT_2 * k1.d}, torque, g);
-  const S4 k3 = dsdt_group<G>(S4{s.a + DT_2 * k2.a, s.b + DT_2 * k2.b, s.c + DT_2 * k2.c, s.d + DT_2 * k2.d}, torque, g);
-  const S4 k4 = dsdt_group<G>(S4{s.a + DT * k3.a, s.b + DT * k3.b, s.c + DT * k3.c, s.d + DT * k3.d}, torque, g);
-  const float na = s.a + DT_6 * (((k1.a + 2.0f * k2.a) + 2.0f * k3.a) + k4.a);
-  const float nb = s.b + DT_6 * (((k1.b + 2.0f * k2.b) + 2.0f * k3.b) + k4.b);
-  const float nc = s.c + DT_6 * (((k1.c + 2.0f * k2.c) + 2.0f * k3.c) + k4.c);
-  const float nd = s.d + DT_6 * (((k1.d + 2.0f * k2.d) + 2.0f * k3.d) + k4.d);
-  s.a = wrap(na);
-  s.b = wrap(nb);
-  s.c = clip(nc, -MAX_VEL_1, MAX_VEL_1);
-  s.d = clip(nd, -MAX_VEL_2, MAX_VEL_2);
 }
 
 // The fused ES rollout's body (es_rollout.h): Gym's observation, the 6-H-3 tanh policy with
@@ -207,10 +239,7 @@ struct RolloutBody {
     float torque = -1.0f, best = l[0];
     if (l[1] > best) { torque = 0.0f; best = l[1]; }
     if (l[2] > best) { torque = 1.0f; }
-    if constexpr (G == 1)
-      rk4(s, torque);
-    else
-      rk4_group<G>(s, torque, g);
+    rk4<G>(s, torque, g);
     t = trig<G>(s, g);
     return (-t.cos_a) - t.cos_ab > 1.0f;  // terminal(s)
   }

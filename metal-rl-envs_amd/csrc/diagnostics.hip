@@ -109,7 +109,7 @@ __global__ __launch_bounds__(kBlock) void arith_check_kernel(uint64_t first, uin
     const double e_recip = fabs(__builtin_fma(-(double)x, recip_normal(x), 1.0));
     if (!(e_root <= 0x1p-51) || !(e_recip <= 0x1p-51)) atomicAdd(&counts[3], 1ull);
   }
-  if (fabsf(x) <= 1.5f) {
+  if (fabsf(x) <= ac::kMassRange) {
     const float d1 = ac::mass_d1(x), d2 = ac::mass_d2(x), r = __builtin_amdgcn_rcpf(d1);
     if (!same_bits(ac::mass_quotient(d2, d1, r), d2 / d1) || !same_bits(ac::mass_quotient(d2 * d2, d1, r), (d2 * d2) / d1))
       atomicAdd(&counts[3], 1ull);

@@ -43,6 +43,48 @@ def test_step_bit_exact_at_the_benchmark_size(dev):
     assert 0 < edone.sum() < len(edone)
 
 
+def _far_states(n, seed):
+    """random_batch with theta2 of 1e18 to 1e20: det_sincos's reduction has no digits left there and
+    its cosine, which the mass matrix is a function of, takes any size; past 4e19 the square of
+    an entry overflows, and the results stay finite."""
+    state, action = random_batch(n, seed=seed)
+    r = np.random.default_rng(seed + 1)
+    state[1] = (10.0 ** r.uniform(18, 20, n) * r.choice([-1, 1], n)).astype(np.float32)
+    assert (np.abs(oa.detmath.cos(state[1])) > 4e19).sum() > n // 4
+    return state, action
+
+
+def test_step_with_angles_past_the_sincos_reduction(dev):
+    from hipenvs import acrobot
+
+    state, action = _far_states(5000, seed=40)
+    with np.errstate(all="ignore"):
+        want = oa.step(state, action, seed=11)
+    assert np.isfinite(want[0]).all()
+    acrobot.reseed(10)
+    got = acrobot.step(torch.from_numpy(state).to(dev), torch.from_numpy(action).to(dev))
+    for g, w in zip(got, want):
+        np.testing.assert_array_equal(to_np(g), w)
+
+
+def test_rollout_with_angles_past_the_sincos_reduction(dev):
+    """The same start states in the rollout, in its 16-, 4- and 1-lane forms: five steps, of which
+    the first is out of range (angles are wrapped after it)."""
+    from hipenvs import acrobot_rollout
+
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    n = 128 * cus + 1
+    state, _ = _far_states(n, seed=41)
+    theta = (np.random.default_rng(5).standard_normal((n, 10 * 8 + 3)) * 0.5).astype(np.float32)
+    with np.errstate(all="ignore"):
+        want = oa.rollout_steps(state, theta, 8, 5)
+    assert len(np.unique(want)) > 3
+    dstate, dtheta = torch.from_numpy(state).to(dev), torch.from_numpy(theta).to(dev)
+    for m in (n, 128 * cus, 16 * cus):
+        got = acrobot_rollout.rollout_steps(dstate[:, :m].contiguous(), dtheta[:m], 8, 5)
+        np.testing.assert_array_equal(to_np(got), want[:m])
+
+
 def test_reset_matches_counter_rng(dev):
     from hipenvs import acrobot
 
