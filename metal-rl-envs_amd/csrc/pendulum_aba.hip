@@ -81,7 +81,10 @@ __device__ __forceinline__ void accelerations_with(const float* th, const float*
     }
   }
   // inward: articulated inertia A and bias P of the current link, folded into the parent
-  // (pendulum_aba_np.py:51-82)
+  // (pendulum_aba_np.py:51-82). A pivot D is at least 1, a link's own inertia plus what it
+  // carries, for angles up to about 2^50. Past them det_sincos leaves [-1, 1] and D can be 0 or
+  // infinite: A0 * A0 / D is NaN then, and with it the parent's inertia and every acceleration,
+  // whatever the reciprocal, so recip_normal serves.
   {
     float A0 = 1.0f, A1 = 0.0f, A2 = 1.0f, A3 = 1.0f, A4 = 0.0f, A5 = 1.0f;
     float P0, P1, P2;
@@ -94,7 +97,7 @@ __device__ __forceinline__ void accelerations_with(const float* th, const float*
       uu[i] = (i == 0 ? torque : 0.0f) - P0;
       if (i == 0) break;
       const float D = A0;
-      const double rD = recip_normal(D);  // D >= 1: a link's own inertia plus what it carries
+      const double rD = recip_normal(D);
       const float I0 = A0 - div(A0 * A0, D, rD), I1 = A1 - div(A0 * A1, D, rD), I2 = A2 - div(A0 * A2, D, rD);
       const float I3 = A3 - div(A1 * A1, D, rD), I4 = A4 - div(A1 * A2, D, rD), I5 = A5 - div(A2 * A2, D, rD);
       const float qd = om[i] - om[i - 1];
@@ -140,7 +143,9 @@ __device__ __forceinline__ void accelerations_with(const float* th, const float*
       const float ap0 = aw;
       const float ap1 = (c * ax + s * xy) + c1;
       const float ap2 = ((-s) * ax + c * xy) + c2;
-      const float qdd = div(uu[i] - ((U0[i] * ap0 + U1[i] * ap1) + U2[i] * ap2), U0[i], recip_normal(U0[i]));
+      // the root's pivot divides nothing before this, so it may be 0 with finite U and u
+      const double rU = (i == 0) ? recip(U0[i]) : recip_normal(U0[i]);
+      const float qdd = div(uu[i] - ((U0[i] * ap0 + U1[i] * ap1) + U2[i] * ap2), U0[i], rU);
       aw = ap0 + qdd;
       ax = ap1;
       ay = ap2;
@@ -514,7 +519,7 @@ __device__ __forceinline__ void staged_inward(const float (&vw)[K], const float 
       sv[i - kStageLinks] = sn_l[(i - kStageLinks) * kBlock];
     }
     const float D = A0;
-    const double rD = recip_normal(D);  // D >= 1: a link's own inertia plus what it carries
+    const double rD = recip_normal(D);
     const float I0 = A0 - div(A0 * A0, D, rD), I1 = A1 - div(A0 * A1, D, rD), I2 = A2 - div(A0 * A2, D, rD);
     const float I3 = A3 - div(A1 * A1, D, rD), I4 = A4 - div(A1 * A2, D, rD), I5 = A5 - div(A2 * A2, D, rD);
     const float c1 = qdv[i] * vy[i], c2 = (-qdv[i]) * vx[i];
@@ -743,7 +748,7 @@ __device__ __forceinline__ void rk4_inward(const float (&vw)[K], const float (&v
       sv[i - kStageLinks] = sn_l[(i - kStageLinks) * kBlock];
     }
     const float D = A0;
-    const double rD = recip_normal(D);  // D >= 1: a link's own inertia plus what it carries
+    const double rD = recip_normal(D);
     const float I0 = A0 - div(A0 * A0, D, rD), I1 = A1 - div(A0 * A1, D, rD), I2 = A2 - div(A0 * A2, D, rD);
     const float I3 = A3 - div(A1 * A1, D, rD), I4 = A4 - div(A1 * A2, D, rD), I5 = A5 - div(A2 * A2, D, rD);
     const float qd = o[i] - o[i - 1];

@@ -27,6 +27,31 @@ def test_accelerations_match_oracle(dev, k):
     np.testing.assert_array_equal(to_np(got), oaba.aba_accelerations(state[:k], state[k:], torque, k))
 
 
+# angles past the range of det_sincos's reduction, whose sines and cosines leave [-1, 1], at which
+# the root's articulated inertia rounds to exactly 0
+ROOT_PIVOT_ZERO = [
+    [2.880969524383545, 4.56531444194345e+16, -5.70906337387479e+16, 2.012966131282739e+16],
+    [-0.20194557309150696, -1.1280371684684595e+17, 1.426235115742167e+17, -1.321864232173568e+17],
+    [-2.7075650691986084, 8.037208378730086e+16, 6.954369813997158e+16, -4.391268193717453e+16,
+     4.420706758557696e+16, -4.158958566637568e+16, -1.0489815093372518e+17, 5.455867750331187e+16],
+]
+
+
+@pytest.mark.parametrize("angles", ROOT_PIVOT_ZERO)
+def test_a_root_pivot_of_zero_divides_as_ieee(dev, angles):
+    """The root's acceleration is infinite there, of the oracle's sign, and not NaN."""
+    from hipenvs import pendulum_aba
+
+    k = len(angles)
+    state = np.concatenate([angles, np.zeros(k)]).astype(np.float32)[:, None]
+    torque = np.ones(1, np.float32)
+    with np.errstate(all="ignore"):
+        want = oaba.aba_accelerations(state[:k], state[k:], torque, k)
+    assert np.isinf(want[0, 0])
+    got = pendulum_aba.Pendulum(k).accelerations(torch.from_numpy(state).to(dev), torch.from_numpy(torque).to(dev))
+    np.testing.assert_array_equal(to_np(got), want)
+
+
 @pytest.mark.parametrize("k", KS)
 def test_rk4_step_matches_oracle(dev, k):
     """test_pendulum_aba.py:44-54's states, every column compared."""
