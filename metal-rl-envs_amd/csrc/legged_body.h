@@ -455,7 +455,9 @@ __device__ __forceinline__ void substep(float (&q)[3 + C], float (&v)[3 + C], co
     }
     asm volatile("" ::: "memory");  // the columns live in LDS until the velocity update
   }
-  // block projected Gauss-Seidel, fixed contact order (legged_np.py:88-93)
+  // block projected Gauss-Seidel, fixed contact order (legged_np.py:88-93). One contact is coupled
+  // to no other: every sweep solves it from the same free velocity, so the first is the result.
+  const int sweeps = C == 1 ? (iters > 0 ? 1 : 0) : iters;
   float lt[C], ln[C];
   ContactBlock blk[C];
 #pragma unroll
@@ -543,7 +545,7 @@ __device__ __forceinline__ void substep(float (&q)[3 + C], float (&v)[3 + C], co
     // from there folds into its only use instead of being shared
     constexpr int kTwin = kGroup == 16 && 4 * C <= kGroup ? 2 * C : 0;
     constexpr int kTwinQ = kGroup == 16 ? 4 : 0;
-    for (int it = 0; it < iters; ++it) {
+    for (int it = 0; it < sweeps; ++it) {
       static_for<C>([&](auto kc) {
         constexpr int k = decltype(kc)::value, s = 2 * k / kGroup;
         float wx = w0x[s];
@@ -586,7 +588,7 @@ __device__ __forceinline__ void substep(float (&q)[3 + C], float (&v)[3 + C], co
       });
     }
   } else {
-    for (int it = 0; it < iters; ++it) {
+    for (int it = 0; it < sweeps; ++it) {
 #pragma unroll
       for (int k = 0; k < C; ++k) {
         float st = 0.0f, sn = 0.0f;

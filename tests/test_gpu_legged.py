@@ -267,6 +267,35 @@ def test_group_tail_equals_static(dev, c, hidden, iters):
         assert ss.max().item() > 8  # members outlived the first chunk
 
 
+@pytest.mark.parametrize("per_cu", [2, 24, 40])
+def test_one_leg_solves_its_contact_once(dev, per_cu):
+    """With one contact every sweep solves the same problem: any number of sweeps gives the first
+    one's result in its time (16 lanes, 8 lanes and one lane per env; all 4,096 sweeps took 170, 220
+    and 53 times as long)."""
+    from hipenvs import legged, legged_rollout
+
+    n = per_cu * torch.cuda.get_device_properties(dev).multi_processor_count
+    theta = torch.from_numpy(_population(2, 1, 8, 0.3, 4)[0]).to(dev)
+    state = legged.Legged(1).reset(n, seed=3, device=dev)
+
+    def scores_and_ms(iters):
+        times = []
+        for _ in range(4):  # the first warms up
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            out = legged_rollout.evaluate(state, theta, 8, 60, 1, iters)
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end))
+        return out, min(times[1:])
+
+    one, one_ms = scores_and_ms(1)
+    many, many_ms = scores_and_ms(4096)
+    assert torch.equal(one, many)
+    assert many_ms < 4 * one_ms
+    assert not torch.equal(one, legged_rollout.evaluate(state, theta, 8, 60, 1, 0))  # no sweep: no contact
+
+
 @pytest.mark.parametrize("c,hidden", [(1, 64), (2, 4), (2, 32)])
 def test_small_tail_bounds(dev, c, hidden):
     """At C <= 2, populations and evaluations past 16 per CU run in 8-lane groups up to 32 per
