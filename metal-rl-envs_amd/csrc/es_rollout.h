@@ -210,6 +210,14 @@ constexpr int kLdsFloats = 16 * Policy<Body, H, 4>::kRow > 4 * Policy<Body, H, 1
                                ? 16 * Policy<Body, H, 4>::kRow
                                : 4 * Policy<Body, H, 16>::kRow;
 
+// Whether the form runs populations of any size with more threads than members: at H = 64, 4 lanes
+// per member past the 16-lane bound. A grid's x has to stay below 2^32 threads (past that the
+// launch reports no error and runs the remainder of the division), which 2^30 members would
+// reach: their blocks spread over rows of kMaxBlocksX. (An evaluation of 2^30 envs holds 21 GB.)
+template <int H, int G>
+constexpr bool kRowedGrid = G == 4 && H > 32;
+constexpr int64_t kMaxBlocksX = (1LL << 26) - 1;
+
 // G lanes per member at the start. member_stride D for a population, 0 for one policy shared by
 // every env (the greedy evaluation).
 template <class Body, int H, int G>
@@ -219,7 +227,9 @@ __global__ __launch_bounds__(64, (Body::template kMinWaves<H, G>)) void rollout_
   __shared__ __align__(16) float lds[kLdsFloats<Body, H>];
   __shared__ Slot slots[16];
   constexpr int M = 64 / G;
-  const int64_t i = (int64_t)blockIdx.x * M + (int)threadIdx.x / G;
+  int64_t block = blockIdx.x;
+  if constexpr (kRowedGrid<H, G>) block += (int64_t)blockIdx.y * gridDim.x;
+  const int64_t i = block * M + (int)threadIdx.x / G;
   int64_t m = i < p ? i : p - 1;  // a group past p steps member p - 1, unused
   State4 x{state[m], state[p + m], state[2 * p + m], state[3 * p + m]};
   int32_t t = 0;
@@ -239,8 +249,10 @@ template <class Body, int H, int G>
 int launch(const float* state, const float* theta, int64_t member_stride, int64_t p, int32_t horizon, float sign,
            float* out, hipStream_t s) {
   constexpr int M = 64 / G;
-  hipLaunchKernelGGL((rollout_kernel<Body, H, G>), dim3((unsigned)((p + M - 1) / M)), dim3(64), 0, s, state, theta,
-                     member_stride, p, horizon, sign, out);
+  const int64_t blocks = (p + M - 1) / M;
+  const int64_t rows = kRowedGrid<H, G> ? (blocks + kMaxBlocksX - 1) / kMaxBlocksX : 1;
+  hipLaunchKernelGGL((rollout_kernel<Body, H, G>), dim3((unsigned)((blocks + rows - 1) / rows), (unsigned)rows),
+                     dim3(64), 0, s, state, theta, member_stride, p, horizon, sign, out);
   return launch_status();
 }
 

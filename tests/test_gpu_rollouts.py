@@ -133,6 +133,29 @@ def test_shared_policy_takes_every_starting_form(dev):
         assert torch.equal(got, want)
 
 
+def test_shared_policy_past_2_to_the_30_envs(dev):
+    """At H = 64 an evaluation runs 4 lanes per env; one of more than 2^30 envs (21 GB of states and
+    scores) needs more threads than a grid's x can have."""
+    from hipenvs import cartpole_rollout
+
+    block, n = 1 << 20, (1 << 30) + 17
+    part = oc.reset(block, seed=6)
+    part[2, ::5] = 0.207  # these fall within the two steps
+    part[3, ::5] = 0.2
+    part = torch.from_numpy(part).to(dev)
+    state = torch.empty((4, n), dtype=torch.float32, device=dev)
+    for a in range(0, n, block):
+        state[:, a:a + block] = part[:, :n - a]
+    theta = torch.from_numpy(population(2, 7 * 64 + 2, 3, scale=0.4)[0]).to(dev)
+    want = cartpole_rollout.evaluate(part, theta, 64, 2)
+    assert len(want.unique()) > 1
+    got = cartpole_rollout.evaluate(state, theta, 64, 2)
+    del state
+    assert torch.equal(got[1 << 30:], want[:17])
+    for a in range(0, 1 << 30, 1 << 28):
+        assert bool((got[a:a + (1 << 28)].view(-1, block) == want).all())
+
+
 def test_config2_cartpole_population(dev):
     """P = 4,096 antithetic members (sigma 0.1) around theta0 = 0.1 N(0,1), H = 32, horizon 500."""
     from hipenvs import cartpole_rollout
