@@ -56,15 +56,17 @@ def test_acrobot_rollout_matches_oracle(dev, hidden):
 
 @pytest.mark.parametrize("hidden", [8, 32])
 def test_large_populations_one_member_per_lane(dev, hidden):
-    """Populations above the 16-lane form's bound start with fewer lanes per member; both bodies,
-    bit for bit against the oracle."""
+    """Populations past the 4-lane form's bound start with one lane per member; both bodies, bit for
+    bit against the oracle."""
     from hipenvs import acrobot_rollout, cartpole_rollout
 
-    p = 20_000
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    p = (256 if hidden >= 16 else 128) * cus + 1
     theta = population(p, 7 * hidden + 2, 100 + hidden, scale=0.5)
     state = oc.reset(p, seed=5)
     got = cartpole_rollout.rollout_steps(torch.from_numpy(state).to(dev), torch.from_numpy(theta).to(dev), hidden, 150)
     np.testing.assert_array_equal(to_np(got), oc.rollout_survived(state, theta, hidden, 150))
+    p = 128 * cus + 1
     theta = population(p, 10 * hidden + 3, 200 + hidden, scale=0.5)
     state = oa.reset(p, seed=6)
     got = acrobot_rollout.rollout_steps(torch.from_numpy(state).to(dev), torch.from_numpy(theta).to(dev), hidden, 60)
@@ -72,18 +74,31 @@ def test_large_populations_one_member_per_lane(dev, hidden):
 
 
 def _mixed_population(body, p, hidden, seed):
-    """Half the members balance (CartPole) or are as drawn, half are wild, shuffled: a wave's
-    members fail at many different steps, so it passes through every lane-group form."""
+    """(theta, state, horizon) of members that end at many different steps, so that a wave passes
+    through its lane-group forms in mid-episode. CartPole: wild policies, of which one in twelve
+    balances. Acrobot: wild policies from fast start states, most of which swing past the goal's
+    height sooner or later (from rest hardly any does)."""
     i, o = (4, 2) if body == "cartpole" else (6, 3)
     r = np.random.default_rng(seed)
     theta = (r.standard_normal((p, i * hidden + hidden + hidden * o + o)) * 0.3).astype(np.float32)
-    if body == "cartpole":
-        good = r.random(p) < 0.5
-        theta[good] *= np.float32(0.2)
-        theta[good, :4 * hidden] += np.repeat(np.array([0.1, 0.4, 4.0, 1.2], np.float32), hidden)
-        theta[good, 5 * hidden:7 * hidden:2] -= np.float32(1.0)
-        theta[good, 5 * hidden + 1:7 * hidden:2] += np.float32(1.0)
-    return theta
+    if body == "acrobot":
+        state = np.stack([r.uniform(-np.pi, np.pi, p), r.uniform(-np.pi, np.pi, p), r.normal(0, 6, p),
+                          r.normal(0, 12, p)]).astype(np.float32)
+        return theta, state, 90
+    good = r.random(p) < 1 / 12
+    theta[good] *= np.float32(0.2)
+    theta[good, :4 * hidden] += np.repeat(np.array([0.1, 0.4, 4.0, 1.2], np.float32), hidden)
+    theta[good, 5 * hidden:7 * hidden:2] -= np.float32(1.0)
+    theta[good, 5 * hidden + 1:7 * hidden:2] += np.float32(1.0)
+    return theta, oc.reset(p, seed=11), 150
+
+
+def _share_narrowing(scores, horizon, members, left):
+    """Of the blocks of `members` consecutive scores (a wave's members), the share that comes down to
+    `left` live ones after the first step and before the horizon."""
+    s = np.sort(scores[:len(scores) // members * members].reshape(-1, members), axis=1)
+    at = s[:, members - left - 1]  # the step that ends all but the `left` longest
+    return ((at > 0) & (at < horizon)).mean()
 
 
 # members per CU at which the starting form changes (16, 4, 1 lanes per member), per body and H
@@ -95,23 +110,25 @@ _FORM_BOUNDS = {("cartpole", 4): (32, 128), ("cartpole", 32): (32, 256), ("cartp
 def test_every_starting_form_gives_the_same_scores(dev, body, hidden):
     """Populations just past each bound of the launch rule (ragged last waves) against the same
     members run in slices small enough for the 16-lane form, which the tests above pin to the
-    oracle: every member's score equal, whatever forms its wave went through."""
+    oracle: every member's score equal, whatever forms its wave went through. Nearly every wave
+    regroups in mid-episode: from one lane at 16 members left, from 4 lanes at 4."""
     from hipenvs import acrobot_rollout, cartpole_rollout
 
     mod = cartpole_rollout if body == "cartpole" else acrobot_rollout
-    reset = oc.reset if body == "cartpole" else oa.reset
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
     b16, b4 = _FORM_BOUNDS[body, hidden]
     p = (b4 or 2 * b16) * cus + 37
-    horizon = 150 if body == "cartpole" else 90
-    theta = torch.from_numpy(_mixed_population(body, p, hidden, 7 + hidden)).to(dev)
-    state = torch.from_numpy(reset(p, seed=11)).to(dev)
+    theta, state, horizon = _mixed_population(body, p, hidden, 7 + hidden)
+    theta, state = torch.from_numpy(theta).to(dev), torch.from_numpy(state).to(dev)
     want = torch.cat([mod.rollout_steps(state[:, a:a + 4001].contiguous(), theta[a:a + 4001], hidden, horizon)
                       for a in range(0, p, 4001)])
     for n in (p, b16 * cus + 1, b16 * cus):
         got = mod.rollout_steps(state[:, :n].contiguous(), theta[:n], hidden, horizon)
         assert torch.equal(got, want[:n]), n
-    assert len(want.unique()) > 3  # members ended at many different steps
+    scores = to_np(want)
+    assert len(np.unique(scores)) > 40
+    for members, left, share in ((64, 16, 0.9), (16, 4, 0.9), (64, 4, 0.15)):  # of waves: measured 1, 0.98, 0.25
+        assert _share_narrowing(scores, horizon, members, left) > share, (members, left)
     one = mod.rollout_steps(state[:, :1].contiguous(), theta[:1], hidden, horizon)
     assert torch.equal(one, want[:1])
     for h in (0, 1):  # nothing to step; the horizon reached in the first form
