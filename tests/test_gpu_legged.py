@@ -74,7 +74,8 @@ def test_step_forms_give_the_same_bits(dev, c, iters, assist):
     """Batches at each bound of the lane-group rule (16 and 64 envs per CU), with ragged last
     workgroups, against the one-lane kernel (which the tests above pin to the oracle) stepping
     the same envs in a larger batch: the same state, reward and flag for every env, NaN for
-    NaN."""
+    NaN. (C = 1 has the one-lane form alone: there the batch's size changes nothing; its group
+    forms and the 8- and 16-lane ones at C = 2 are in the next test.)"""
     from hipenvs import legged
 
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
@@ -93,6 +94,34 @@ def test_step_forms_give_the_same_bits(dev, c, iters, assist):
             zeros = want[..., :m] == 0  # and the sign of a zero
             np.testing.assert_array_equal(np.signbit(got[zeros].astype(np.float32)),
                                           np.signbit(want[..., :m][zeros].astype(np.float32)))
+
+
+@pytest.mark.parametrize("c", [1, 2])
+@pytest.mark.parametrize("iters", [1, 8])
+def test_rollout_forms_give_the_same_bits_from_rough_states(dev, c, iters):
+    """The same states at C <= 2 in the forms that only rollouts and evaluations have: 16 lanes up to
+    16 members per CU, 8 up to 32, and past them chunks of 4 lanes per member while 32 to 64 of
+    them per CU are left, each against one lane per member."""
+    from hipenvs import legged_rollout
+
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    hidden, horizon, chunk = 8, 14, 4
+    n = 70 * cus
+    state = torch.from_numpy(_rough_states(c, n, seed=50 + c)[0]).to(dev)
+    theta = torch.from_numpy(_population(n, c, hidden, 0.3, 13)).to(dev)
+    for p in (16 * cus, 32 * cus, n):
+        s, th = state[:, :p].contiguous(), theta[:p]
+        got = legged_rollout.rollout(s, th, hidden, horizon, c, schedule="chunked", chunk_steps=chunk, iters=iters)
+        want = legged_rollout.rollout(s, th, hidden, horizon, c, schedule="rows", iters=iters)
+        for g, w in zip(got, want):
+            np.testing.assert_array_equal(to_np(g), to_np(w))
+    left = int((want[1] > chunk).sum())  # after the whole population's first chunk
+    assert 32 * cus < left <= 64 * cus, left
+    assert torch.isnan(want[0]).any()
+    scores = to_np(legged_rollout.evaluate(state, theta[0], hidden, horizon, c, iters))  # one lane per env
+    for m in (16 * cus, 32 * cus):
+        got = legged_rollout.evaluate(state[:, :m].contiguous(), theta[0], hidden, horizon, c, iters)
+        np.testing.assert_array_equal(to_np(got), scores[:m])
 
 
 @pytest.mark.parametrize("c", [1, 2, 4])
