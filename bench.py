@@ -25,7 +25,9 @@ launch (FETCH_SIZE + WRITE_SIZE, scaled by a copy of known size).
 and op order with np.sin/np.cos, one process) at the same N for a bounded
 sample of about `--cpu-seconds` seconds on this host.
 
-`extra` holds the rest of the workload list, measured in the same run:
+`extra` holds the rest of the workload list, measured in the same run, in the line as rates,
+times and fractions of four digits (the line stays below LINE_CHARS characters, which a log's
+tail keeps whole) and in full in the file that `--extra-out` names:
 * `legged4_es_rollout`, `legged2_es_rollout`: the fused legged ES rollout at
   N = 262,144 members, C = 4 legs (quadruped) and C = 2 (biped), H = 64, sigma 0.03
   antithetic around theta0 = 0.1 N(0, 1), alive bonus 1 + forward velocity,
@@ -70,7 +72,7 @@ sample of about `--cpu-seconds` seconds on this host.
   one's do;
 
 Usage: python bench.py [--gpus 1] [--steps 1000] [--warmup 16] [--repeats 3] [--sweep] [--skip-cpu]
-                      [--only cartpole|legged|aba|steps|generation]
+                      [--only cartpole|legged|aba|steps|generation] [--extra-out FILE]
 """
 
 import argparse
@@ -86,6 +88,12 @@ for p in (str(ROOT), str(ROOT / "metal-rl-envs_amd")):
     if p not in sys.path:
         sys.path.insert(0, p)
 
+LINE_CHARS = 7600
+# what the line keeps of a workload's record, beside the names of its parts
+LINE_KEYS = {"env_steps_per_s", "us_per_launch", "us_per_iteration", "wall_s", "rollout_s", "ms", "generation_ms",
+             "peak_alloc_gib", "p_x_horizon_per_s", "steps_taken_per_s", "inkernel_actions_env_steps_per_s",
+             "array_actions_env_steps_per_s", "copy_us_per_launch", "step_resident_us_per_launch", "crossover_n",
+             "crossover_n_sampler_and_step", "speedup_vs_cpu", "speedup_vs_cpu_s8", "speedup_p_x_horizon_vs_cpu"}
 METRIC = "env-steps/s at N=2^18 (CartPole, legged-4c ES rollout); % HBM/VALU roofline"
 HBM_PEAK_GBS = 8000.0
 FP32_PEAK_TFLOPS = 157.3           # MI355X FP32 vector, packed (published)
@@ -140,6 +148,7 @@ def parse_args():
     p.add_argument("--legged-horizon", type=int, default=1000)
     p.add_argument("--sweep", action="store_true", help="also run the CartPole N = 2^0..2^24 sweep")
     p.add_argument("--sweep-out", default=None)
+    p.add_argument("--extra-out", default=None, help="write the full records of `extra` to this file")
     p.add_argument("--copy-mib", type=int, default=0,
                    help="first run a plain device-to-device copy of this many MiB three times (a known-size "
                         "kernel that scales hardware byte counters)")
@@ -1102,6 +1111,39 @@ def bench_step_bodies(dev, steps=1000, n=65536, ks=(2, 4, 8, 16)):
     return out
 
 
+def brief(rec):
+    """A workload's record as the line carries it: LINE_KEYS to four digits, each roofline as its
+    fraction, a sweep as its sampler + step rates by N."""
+    if isinstance(rec, list):
+        if rec and isinstance(rec[0], dict) and "sampled" in rec[0]:
+            return {str(r["n"]): float(f"{r['sampled']:.4g}") for r in rec}
+        return [brief(r) for r in rec if isinstance(r, dict)]
+    out = {}
+    for k, v in rec.items():
+        if k == "roofline":
+            out["frac"] = float(f"{v['frac']:.4g}")
+        elif k != "cpu_baseline" and isinstance(v, (dict, list)):
+            part = brief(v)
+            if part:
+                out[k] = part
+        elif k in LINE_KEYS and isinstance(v, (int, float)):
+            out[k] = float(f"{v:.4g}")
+    return out
+
+
+def result_line(line):
+    """The JSON line, below LINE_CHARS characters whatever was measured: past them the longest
+    entries of `extra` leave it."""
+    line = dict(line, extra={k: brief(v) for k, v in line["extra"].items()})
+    text = json.dumps(line)
+    while len(text) >= LINE_CHARS and line["extra"]:
+        longest = max(line["extra"], key=lambda k: len(json.dumps(line["extra"][k])))
+        log(f"extra.{longest} left out of the line (over {LINE_CHARS} characters)")
+        del line["extra"][longest]
+        text = json.dumps(line)
+    return text
+
+
 def main():
     args = parse_args()
     if args.gpus != 1:
@@ -1227,7 +1269,9 @@ def main():
         "dtype": "fp32", "data": "synthetic (counter-RNG states and actions, seeded Gaussian ES populations)",
         "config": config, "roofline": roofline, "cpu_baseline": cpu, "extra": extra,
     }
-    print(json.dumps(line), flush=True)
+    if args.extra_out:
+        Path(args.extra_out).write_text(json.dumps(extra, indent=1))
+    print(result_line(line), flush=True)
 
 
 if __name__ == "__main__":
