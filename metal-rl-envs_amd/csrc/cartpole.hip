@@ -170,8 +170,10 @@ struct RolloutBody {
 //   H = 64: P = 8,192 563 / 916; 65,536 3,153 / 2,378 (its 450 weights leave one lane one wave
 //           per SIMD: 2,864)
 // Populations early in training, whose waves narrow as their members fail, are within 10 %
-// between the forms at these bounds. (One member per lane to the end, as before: P = 262,144,
-// H = 32 early in training 2,844 us, now 402; trained 5,147, now 4,133.)
+// between the forms at these bounds. One member per lane to the end, with the same arithmetic,
+// takes 3,899 us at P = 262,144, H = 32 early in training and 3,891 trained, this kernel 574 and
+// 4,135: the check for finished members and the registers of the other forms cost a population
+// that runs to the horizon 6 %.
 constexpr int kGroup16PerCu = 32;
 template <int H>
 constexpr int kGroup4PerCu = H >= 16 ? 256 : 128;

@@ -491,7 +491,8 @@ __device__ __forceinline__ void substep(float (&q)[3 + C], float (&v)[3 + C], co
     // cone's width); broadcasts fold into their uses (v_sub, v_mul, v_add, v_max with a DPP
     // operand). 16 lanes, C = 4: about 164 instructions a sweep (145 VALU) where per-pair coupling
     // terms, separate broadcasts and a masked clamp and gate took 203 (182 VALU). Quadruped ES
-    // rollout at P = 262,144, H = 64, 1,000 steps, 8 sweeps 30.6 -> 27.1 ms; generation at
+    // rollout at P = 262,144, H = 64, 1,000 steps, 8 sweeps 30.6 -> 27.1 ms for one population
+    // (1.07x to 1.13x, as many members last); generation at
     // P = 1,024, H = 16, every member standing for 500 steps 20.2 -> 17.5 ms (17.05 with a row of the
     // setup per lane too, kRows).
     const bool edge = (g == 2 || g == 3);

@@ -69,7 +69,8 @@ def test_sqrt_and_recip_match_ieee_for_every_float32(dev):
     """The kernels' square root (float64 reciprocal square root estimate, one Newton step,
     rounded to float32) and float64 reciprocal (hardware estimate, two Newton steps) against
     IEEE sqrtf and 1.0 / (double)x, over all 2^32 float32 bit patterns, in 16 launches of
-    2^28. The Cholesky pivots and the shared-reciprocal divisions rest on both."""
+    2^28. The IEEE form of the Cholesky pivots takes the root, the shared-reciprocal divisions the
+    reciprocal."""
     counts = torch.zeros(2, dtype=torch.int64, device=dev)
     step = 1 << 28
     for first in range(0, 1 << 32, step):
