@@ -697,14 +697,17 @@ __device__ __forceinline__ void substep_exact(float (&q)[3 + C], float (&v)[3 + 
   }
   DivRecip fast;
   substep<C, DivRecip, 0, kHopperSum, kStage>(q, v, tq, iters, assist, assist_damping, fast, stage);
-  if (fast.saw_subnormal() || (v[2] != v[2] && finite_angles<C>(q0))) {
+  const bool nan = v[2] != v[2];
+  if (fast.saw_subnormal() | nan) {  // one branch on the ordinary path
+    if (fast.saw_subnormal() || finite_angles<C>(q0)) {
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-      q[i] = q0[i];
-      v[i] = v0[i];
+      for (int i = 0; i < N; ++i) {
+        q[i] = q0[i];
+        v[i] = v0[i];
+      }
+      DivIEEE ieee;
+      substep<C, DivIEEE, 0, kHopperSum, kStage>(q, v, tq, iters, assist, assist_damping, ieee, stage);
     }
-    DivIEEE ieee;
-    substep<C, DivIEEE, 0, kHopperSum, kStage>(q, v, tq, iters, assist, assist_damping, ieee, stage);
   }
 }
 
@@ -725,7 +728,7 @@ __device__ __forceinline__ void substep_exact_group(float (&q)[3 + C], float (&v
   DivRecip fast;
   substep<C, DivRecip, G>(q, v, tq, iters, assist, assist_damping, fast, xs, g, xd);
   const bool nan = v[2] != v[2];
-  if (__any(live && (fast.saw_subnormal() || nan)) &&  // lanes of finished members step on, unused
+  if (__any(live & (fast.saw_subnormal() | nan)) &&  // lanes of finished members step on, unused
       __any(live && (fast.saw_subnormal() || (nan && finite_angles<C>(q0))))) {
 #pragma unroll
     for (int i = 0; i < N; ++i) {
